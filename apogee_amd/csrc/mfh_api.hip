@@ -616,6 +616,11 @@ extern "C" int mfh_set_tuning(mfh_ctx *ctx, const char *key, long value) {
     c->big_chunk_bytes = (long long)value << 20;
     return 0;
   }
+  if (!strcmp(key, "wide")) {
+    if (value < 0 || value > 2) return fail("wide must be 0 (by the pair count), 1 (always) or 2 (never)");
+    c->wide = (int)value;
+    return 0;
+  }
   if (!strcmp(key, "coarse_rpw")) {
     if (value != 1 && value != 2) return fail("coarse_rpw must be 1 or 2");
     c->coarse_rpw = (int)value;

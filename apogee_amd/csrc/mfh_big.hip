@@ -1,13 +1,19 @@
-// Flat filter for n = 32768 and 65536: a four-step split across two kernels.
+// Flat filter for n >= 32768 across two kernels, columns and rows.
 //
-// A length-n transform no longer fits one workgroup's LDS (256/512 KiB), so
-// n = N1 x 256 (N1 = 128 or 256) with f = f1 + N1 f2 and k = k2 + 256 k1:
+// n >= 131072: a four-step split.  A length-n transform does not fit one
+// workgroup, so n = N1 x 256 with f = f1 + N1 f2 and k = k2 + 256 k1:
 //   Y[f1][k2] = w_n^(f1 k2) sum_f2 P[f1 + N1 f2] w_256^(f2 k2)     kernel A
 //   z[k2 + 256 k1] = sum_f1 Y[f1][k2] w_N1^(f1 k1)                 kernel B
+// n = 32768 and 65536 (RF = n / 4096), for calls of few pairs: the four passes
+// of the one-workgroup transform (mfh_wide.hip), the first two in kernel A
+// (256 columns of 16 RF points), the last two in kernel B (16 RF rows of 256
+// points), with the same arithmetic and so the same bits.  Spread over many
+// workgroups, one pair takes 14 us instead of 33 at n = 65536; from about
+// a hundred pairs on the scratch round trip costs more than it gives.
 // Kernel A forms the product D*conj(T) on load, runs 256-point inverse FFTs
 // over 16 columns per workgroup and writes Y k2-major to scratch (each
-// 16-lane group writes 128 contiguous bytes).  Kernel B gives each pair one
-// workgroup that walks all k2 in groups, runs N1-point inverse FFTs, and keeps
+// 16-lane group writes 128 contiguous bytes).  Kernel B gives each pair a few
+// workgroups that walk k2 in groups, run the row transforms, and keep
 // a per-bin (key, value) table in LDS: keys rise by ds_max_u64, and after
 // each group the lane holding the bin's key writes its value, so the table
 // always pairs the largest |z|^2 (lowest lag among equals) with its own z.
@@ -29,6 +35,18 @@ namespace mfh {
 
 namespace {
 
+// ROWS rows of ROW points; columns of ROWS points, CT threads each.  RF > 0:
+// the passes of the one-workgroup transform of n = 4096 RF.
+template <int N1, int RF_ = 0>
+struct BigShape {
+  static constexpr int RF = RF_;
+  static constexpr int ROWS = RF ? 16 * RF : 256;
+  static constexpr int ROW = RF ? 256 : N1;
+  static constexpr int N = ROWS * ROW;
+  static constexpr int CT = ROWS / 16;
+  static constexpr int COL_STRIDE = FlatShape<ROWS>::XCH + 1;  // see kColStride; 137 for 128 points
+};
+
 struct BigArgs {
   const cf *data, *tmpl;
   long long data_stride, tmpl_stride;
@@ -36,9 +54,10 @@ struct BigArgs {
   long long p0;         // first pair (tiled) or list position (list) of this chunk
   const int2 *list;     // list mode
   const int *list_count;
+  int *hint;            // if set, the first workgroup stores the list length there (host-mapped)
   const long long *list_ooff;  // list mode: output element offset per pair
-  cf *scratch;          // [chunk pair][256][N1]
-  const cf *tw256, *twN1;  // Stockham tables of the two lengths
+  cf *scratch;          // [chunk pair][ROWS][ROW]
+  const cf *twCol, *twRow;  // Stockham tables of the column and the row passes
   const cf *rootH, *rootL; // w_N1^h (h < N1) and w_n^l (l < 256)
   int nsplit;               // rows workgroups per pair (gridDim.y of the rows kernel)
   uint64_t *pkey;           // nsplit > 1: per-part bin tables [pair][part][nb]
@@ -101,59 +120,86 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
 // The pair's rows and its Y block are wave-uniform, so loads and stores go
 // through buffer descriptors: one vector offset per thread and the per-u
 // stride as a scalar offset, with no vector address arithmetic per point.
-template <int N1>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) big_cols_kernel(BigArgs a) {
-  constexpr int N = N1 * 256;
+template <class B>
+__global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu(4))) big_cols_kernel(BigArgs a) {
+  constexpr int N = B::N, ROW = B::ROW, CT = B::CT;
   extern __shared__ __align__(16) unsigned char smem[];
   const int s = threadIdx.x & 15;
   const int t = threadIdx.x >> 4;
-  cf *xch = reinterpret_cast<cf *>(smem) + s * kColStride;
-  // The closing twiddle of output k2 = t + 16 u of column f1 splits as
+  cf *xch = reinterpret_cast<cf *>(smem) + s * B::COL_STRIDE;
+  // The four-step closing twiddle of output k2 = t + 16 u of column f1 splits as
   // w_n^(f1 k2) = w_n^(f1 t) * w_n^(16 f1 u): the first factor is one per
   // thread, the second one per (column, u), 256 per workgroup, kept in LDS
   // as bt[17 s + u] (rows of 17: the 16 columns a wave reads in one step
   // fall in distinct banks, its 4 row groups read the same words).
-  cf *bt = reinterpret_cast<cf *>(smem) + 16 * kColStride;
+  cf *bt = reinterpret_cast<cf *>(smem) + 16 * B::COL_STRIDE;
   const long long pl = blockIdx.y;  // pair within the chunk
+  if (a.hint && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.hint = *a.list_count;
   int d = 0, tt = 0;
   const bool valid = big_pair(a, a.p0 + pl, d, tt);  // uniform across the workgroup
   if (!valid) return;                                 // no barrier has run yet
   const int f1 = blockIdx.x * 16 + s;
-  bt[17 * s + t] = big_root(a, 16 * f1 * t);  // u = t; 16 f1 t < n
-  const cf wt = big_root(a, f1 * t);
+  cf wt{1.f, 0.f};
+  if constexpr (!B::RF) {
+    bt[17 * s + t] = big_root(a, 16 * f1 * t);  // u = t; 16 f1 t < n
+    wt = big_root(a, f1 * t);
+  }
   const cf *D = uniform_ptr(a.data + (long long)d * a.data_stride);
   const cf *T = uniform_ptr(a.tmpl + (long long)tt * a.tmpl_stride);
   const __amdgpu_buffer_rsrc_t rd =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<cf *>(D), (short)0, N * (int)sizeof(cf), 0x00020000);
   const __amdgpu_buffer_rsrc_t rt =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<cf *>(T), (short)0, N * (int)sizeof(cf), 0x00020000);
-  const int voff = (f1 + N1 * t) * (int)sizeof(cf);  // element f1 + N1 (t + 16 u) at voff + u * 16 N1 * 8
+  const int voff = (f1 + ROW * t) * (int)sizeof(cf);  // element f1 + ROW (t + CT u) at voff + u * CT ROW * 8
   cf v[16];
 #pragma unroll
   for (int u = 0; u < 16; u++) {
-    const int so = u * 16 * N1 * (int)sizeof(cf);
+    const int so = u * CT * ROW * (int)sizeof(cf);
     const cf x = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rd, voff, so, 0));
     const cf y = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rt, voff, so, 0));
     v[u] = cmul_conj(x, y);
   }
-  inverse_fft<256>(v, t, xch, a.tw256);  // its barriers order the bt stores before the reads
+  inverse_fft<B::ROWS>(v, t, xch, a.twCol);  // its barriers order the bt stores before the reads
   cf *Y = const_cast<cf *>(uniform_ptr(a.scratch + pl * N));
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(Y, (short)0, N * (int)sizeof(cf), 0x00020000);
-  const int yoff = (t * N1 + f1) * (int)sizeof(cf);  // Y[k2][f1], k2 = t + 16 u
+  const int yoff = (t * ROW + f1) * (int)sizeof(cf);  // Y[k2][f1], k2 = t + CT u
 #pragma unroll
   for (int u = 0; u < 16; u++) {
-    const cf w = cmul(wt, bt[17 * s + u]);
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, cmul(v[u], w)), ry, yoff,
-                                          u * 16 * N1 * (int)sizeof(cf), 0);
+    if constexpr (!B::RF) v[u] = cmul(v[u], cmul(wt, bt[17 * s + u]));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[u]), ry, yoff, u * CT * ROW * (int)sizeof(cf), 0);
   }
 }
 
+// The last two passes of the one-workgroup transform over row k of its 16 RF
+// rows: 256 points, thread t holding t + 16 u.  Twiddles as there: the third
+// pass's depend on the row only, the fourth's on k + 16 RF t.
+template <int RF>
+__device__ __forceinline__ void closing_passes(cf *v, int t, int k, cf *xch, const cf *tw) {
+  using L = TwiddleLayout<4096 * RF>;
+  constexpr int p0 = L::NS0 == 1 ? 1 : 0;  // the table of NS = RF
+  const cf *tw3 = tw + L::offset(p0 + 1), *tw4 = tw + L::offset(p0 + 2);
+  cf w[15];
+  power_twiddles(w, tw3[k], tw3[16 * RF + k]);
+#pragma unroll
+  for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
+  dft16(v);
+  stockham_store<256, 16, 1>(v, t, xch);
+  const int j = k + 16 * RF * t;
+  const cf w1 = tw4[j], w4 = tw4[256 * RF + j];
+  __syncthreads();
+  stockham_load<256>(v, t, xch);
+  power_twiddles(w, w1, w4);
+#pragma unroll
+  for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
+  dft16(v);
+}
+
 // Rows: nsplit workgroups per pair (workgroup = pair * nsplit + part), each
-// walking its share of the 256 rows k2, SLOTS rows at a time.  With one part
+// walking its share of the rows k2, SLOTS rows at a time.  With one part
 // the table is the result; with several, each part leaves its (key, value)
 // table, and finish_cell keeps the largest key per bin: in the next chunk's
 // rows launch, or in big_rows_finish_kernel after the last chunk.
-template <int N1>
+template <class B>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
   // the last fin_blocks workgroups finish the previous chunk (its tables
@@ -163,7 +209,8 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     finish_cell(fin, fin_np, (long long)(blockIdx.x - row_blocks) * 256 + threadIdx.x);
     return;
   }
-  using S = FlatShape<N1>;
+  constexpr int ROW = B::ROW, ROWS = B::ROWS;
+  using S = FlatShape<ROW>;
   constexpr int TPT = S::TPT;
   constexpr int SLOTS = S::SLOTS;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -180,11 +227,11 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
   const int nb = (int)a.nb;
   for (int b = threadIdx.x; b < nb; b += 256) bkey[b] = 0ull;
   __syncthreads();
-  const cf *Y = a.scratch + pl * (long long)(N1 * 256);
-  constexpr int G = 256 / SLOTS;  // row groups of the pair
+  const cf *Y = a.scratch + pl * (long long)B::N;
+  constexpr int G = ROWS / SLOTS;  // row groups of the pair
   const int gbeg = part * G / a.nsplit, gend = (part + 1) * G / a.nsplit;
-  const bool whole = a.ws == 0 && a.we == (uint32_t)(N1 * 256);
-  const bool full8 = whole && a.bshift == ilog2(N1 * 256 / 8);
+  const bool whole = a.ws == 0 && a.we == (uint32_t)B::N;
+  const bool full8 = whole && a.bshift == ilog2(B::N / 8);
   FlatArgs fa;  // for bin_of / make_key
   fa.ws = a.ws;
   fa.we = a.we;
@@ -192,17 +239,18 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
   fa.bshift = a.bshift;
   fa.inv_bs = a.inv_bs;
   // the first twiddled pass's twiddles depend on t only: derived once for
-  // all the part's row groups where the registers allow (N1 <= 512)
-  constexpr bool HOIST = N1 <= 512;
+  // all the part's row groups where the registers allow (rows of up to 512 points)
+  constexpr bool HOIST = !B::RF && ROW <= 512;
   cf wf[HOIST ? 15 : 1];
-  if constexpr (HOIST) first_twiddles<N1>(wf, t, a.twN1);
+  if constexpr (HOIST) first_twiddles<ROW>(wf, t, a.twRow);
   for (int g = gbeg; g < gend; g++) {
     const int k2 = g * SLOTS + slot;
     cf v[16];
 #pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = Y[(long long)k2 * N1 + t + TPT * u];
-    inverse_fft<N1, HOIST>(v, t, xch, a.twN1, wf);
-    // thread t holds z[k2 + 256 (t + TPT u)]; lags rise with u.  A wave none
+    for (int u = 0; u < 16; u++) v[u] = Y[(long long)k2 * ROW + t + TPT * u];
+    if constexpr (B::RF > 0) closing_passes<B::RF>(v, t, k2, xch, a.twRow);
+    else inverse_fft<ROW, HOIST>(v, t, xch, a.twRow, wf);
+    // thread t holds z[k2 + ROWS (t + TPT u)]; lags rise with u.  A wave none
     // of whose window lags has |z|^2 above the seed raises no key and records
     // no value, so it skips both steps below (wave-uniform; nonnegative
     // floats order like their bits, and a NaN's bits, above all of them,
@@ -214,7 +262,7 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     } else {
 #pragma unroll
       for (int u = 0; u < 16; u++) {
-        const uint32_t k = (uint32_t)(k2 + 256 * (t + TPT * u));
+        const uint32_t k = (uint32_t)(k2 + ROWS * (t + TPT * u));
         const uint32_t m = __float_as_uint(__builtin_fmaf(v[u].x, v[u].x, v[u].y * v[u].y));
         mloc = (k >= a.ws && k < a.we) ? max(mloc, m) : mloc;
       }
@@ -223,16 +271,16 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     if (!hot) {
     } else if (full8) {
       // n/8 bins over the whole transform: every wave's 64 lanes put u and
-      // u + 1 = 2 rho, 2 rho + 1 in bin rho (their lags span < 256 TPT)
+      // u + 1 = 2 rho, 2 rho + 1 in bin rho (their lags span < ROWS TPT)
       const int lane = threadIdx.x & 63;
       const int k2w = __builtin_amdgcn_readfirstlane(k2);
-      runs8_max_to_bins<256 * TPT>(v, (uint32_t)(k2 + 256 * t), (uint32_t)k2w, lane, a.seed, a.bshift, bkey);
+      runs8_max_to_bins<ROWS * TPT>(v, (uint32_t)(k2 + ROWS * t), (uint32_t)k2w, lane, a.seed, a.bshift, bkey);
     } else {
     uint64_t acc = 0ull;
     int acc_bin = -1;
 #pragma unroll
     for (int u = 0; u < 16; u++) {
-      const uint32_t k = (uint32_t)(k2 + 256 * (t + TPT * u));
+      const uint32_t k = (uint32_t)(k2 + ROWS * (t + TPT * u));
       if (k >= a.ws && k < a.we) {
         const uint64_t key = make_key(v[u], k, a.seed);
         const int b = (int)bin_of(k, fa);
@@ -251,7 +299,7 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     if (hot) {
 #pragma unroll
       for (int u = 0; u < 16; u++) {
-        const uint32_t k = (uint32_t)(k2 + 256 * (t + TPT * u));
+        const uint32_t k = (uint32_t)(k2 + ROWS * (t + TPT * u));
         if (k >= a.ws && k < a.we) {
           const uint64_t key = make_key(v[u], k, a.seed);
           if (key) {
@@ -305,16 +353,16 @@ __global__ void roots_kernel(cf *out, int L, int period) {
 
 constexpr size_t kLds = 160 * 1024;
 
-template <int N1>
+template <class B>
 size_t rows_max_bins() {
-  using S = FlatShape<N1>;
+  using S = FlatShape<B::ROW>;
   return (kLds - (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf)) / (sizeof(uint64_t) + sizeof(cf));
 }
 
-template <int N1>
-int launch_big_n1(Ctx *c, const FlatRun &r) {
-  constexpr int N = N1 * 256;
-  using S = FlatShape<N1>;
+template <class B>
+int launch_big_shape(Ctx *c, const FlatRun &r) {
+  constexpr int N = B::N;
+  using S = FlatShape<B::ROW>;
   BigArgs a;
   a.data = r.data;
   a.tmpl = r.tmpl;
@@ -324,20 +372,25 @@ int launch_big_n1(Ctx *c, const FlatRun &r) {
   a.nt = r.nt;
   a.list = r.list;
   a.list_count = r.list_count;
+  a.hint = r.list ? r.hint : nullptr;
   a.list_ooff = r.list_ooff;
-  a.tw256 = c->twiddles(256);
-  a.twN1 = c->twiddles(N1);
-  const cf *roots = big_roots(c, N1);
-  if (!a.tw256 || !a.twN1 || !roots) return -1;
-  a.rootH = roots;
-  a.rootL = roots + N1;
+  a.twCol = c->twiddles(B::ROWS);
+  a.twRow = c->twiddles(B::RF ? N : B::ROW);
+  if (!a.twCol || !a.twRow) return -1;
+  a.rootH = a.rootL = nullptr;
+  if (!B::RF) {
+    const cf *roots = big_roots(c, B::ROW);
+    if (!roots) return -1;
+    a.rootH = roots;
+    a.rootL = roots + B::ROW;
+  }
   const long long total = r.list ? (long long)r.list_cap : (long long)r.nd * r.nt;
   // scratch in chunks of pairs: at most c->big_chunk_bytes of intermediate data
   const long long chunk = std::max<long long>(1, std::min<long long>(total, c->big_chunk_bytes / ((long long)N * 8)));
   cf *scr = (cf *)c->scratch("big_scratch", (size_t)chunk * N * sizeof(cf));
   if (!scr) return -1;
   a.scratch = scr;
-  const size_t lds_cols = (16 * kColStride + 16 * 17) * sizeof(cf);
+  const size_t lds_cols = (16 * B::COL_STRIDE + 16 * 17) * sizeof(cf);
   const float thr = r.threshold;
   a.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
   a.binsize = (uint32_t)r.binsize;
@@ -345,14 +398,14 @@ int launch_big_n1(Ctx *c, const FlatRun &r) {
   a.bshift = pow2 ? ilog2((int)r.binsize) : -1;
   a.inv_bs = 1.0f / (float)r.binsize;
   const size_t nb_total = (r.we - r.ws + r.binsize - 1) / r.binsize;
-  const size_t maxb = rows_max_bins<N1>();
-  if (!lds_limit((const void *)big_cols_kernel<N1>, c->dev, lds_cols) ||
-      !lds_limit((const void *)big_rows_kernel<N1>, c->dev, kLds))
+  const size_t maxb = rows_max_bins<B>();
+  if (!lds_limit((const void *)big_cols_kernel<B>, c->dev, lds_cols) ||
+      !lds_limit((const void *)big_rows_kernel<B>, c->dev, kLds))
     return -1;
   // rows workgroups per pair: enough for about 1024 workgroups per launch (at
   // least 8, at most one per row group), as long as the per-part tables stay
   // within 64 MiB
-  constexpr int G = 256 / S::SLOTS;
+  constexpr int G = B::ROWS / S::SLOTS;
   const size_t nb_piece = std::min(maxb, nb_total);
   int nsplit = (int)std::min<long long>(G, std::max<long long>(8, (1024 + chunk - 1) / chunk));
   nsplit = 1 << ilog2(nsplit);  // a power of two: parts split the row groups evenly
@@ -385,8 +438,9 @@ int launch_big_n1(Ctx *c, const FlatRun &r) {
       a.pkey = pkey2 + (ci & 1) * part_cells;
       a.pval = pval2 + (ci & 1) * part_cells;
     }
-    hipLaunchKernelGGL(big_cols_kernel<N1>, dim3(N1 / 16, (unsigned)np), dim3(256), lds_cols, c->stream, a);
+    hipLaunchKernelGGL(big_cols_kernel<B>, dim3(B::ROW / 16, (unsigned)np), dim3(16 * B::CT), lds_cols, c->stream, a);
     if (!hip_ok(hipGetLastError(), "big_cols_kernel")) return -1;
+    a.hint = nullptr;
     for (size_t b0 = 0; b0 < nb_total; b0 += maxb) {
       const size_t cnt = std::min(maxb, nb_total - b0);
       a.ws = (uint32_t)(r.ws + b0 * r.binsize);
@@ -397,7 +451,7 @@ int launch_big_n1(Ctx *c, const FlatRun &r) {
       a.out_val = r.out_val + b0;
       const size_t lds = (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf) + cnt * (sizeof(uint64_t) + sizeof(cf));
       const long long row_blocks = np * nsplit;
-      hipLaunchKernelGGL(big_rows_kernel<N1>, dim3((unsigned)(row_blocks + fin_blocks)), dim3(256), lds, c->stream, a,
+      hipLaunchKernelGGL(big_rows_kernel<B>, dim3((unsigned)(row_blocks + fin_blocks)), dim3(256), lds, c->stream, a,
                          fin, fin_np, fin_blocks);
       if (!hip_ok(hipGetLastError(), "big_rows_kernel")) return -1;
       fin_blocks = 0;
@@ -441,13 +495,13 @@ const cf *big_roots(Ctx *c, int n1) {
 
 int launch_big(Ctx *c, size_t n, const FlatRun &r) {
   switch (n) {
-    case 32768: return launch_big_n1<128>(c, r);
-    case 65536: return launch_big_n1<256>(c, r);
-    case 131072: return launch_big_n1<512>(c, r);
-    case 262144: return launch_big_n1<1024>(c, r);
-    case 524288: return launch_big_n1<2048>(c, r);
-    case 1048576: return launch_big_n1<4096>(c, r);
-    default: return fail("transform length %zu is not a four-step length", n);
+    case 32768: return launch_big_shape<BigShape<0, 8>>(c, r);
+    case 65536: return launch_big_shape<BigShape<0, 16>>(c, r);
+    case 131072: return launch_big_shape<BigShape<512>>(c, r);
+    case 262144: return launch_big_shape<BigShape<1024>>(c, r);
+    case 524288: return launch_big_shape<BigShape<2048>>(c, r);
+    case 1048576: return launch_big_shape<BigShape<4096>>(c, r);
+    default: return fail("transform length %zu is not a two-kernel length", n);
   }
 }
 

@@ -68,12 +68,12 @@ struct FlatShape {
   static constexpr int XSTRIDE = TPT < 64 ? XCH + 1 : XCH;
 };
 
-// Four-step column transforms: 16 lanes of a row group serve 16 adjacent
-// columns, each column a 256-point transform with its own exchange buffer.
-// A buffer stride of 273 elements (546 dwords, 34 mod 64) puts the 16 lanes'
-// equal offsets in 16 distinct bank pairs; 272 would fold them onto two.
-// (An even stride, 274, measured 2.8x the bank-conflict cycles of 273 in the
-// columns kernel: the 16 columns are what must spread over the banks.)
+// Column transforms of the two-kernel lengths: 16 lanes of a row group serve 16
+// adjacent columns, each column with its own exchange buffer.  For columns of
+// 256 points a buffer stride of 273 elements (546 dwords, 34 mod 64) puts the
+// 16 lanes' equal offsets in 16 distinct bank pairs; 272 would fold them onto
+// two.  (An even stride, 274, measured 2.8x the bank-conflict cycles of 273 in
+// the columns kernel: the 16 columns are what must spread over the banks.)
 constexpr int kColStride = FlatShape<256>::XCH + 1;
 
 __device__ __forceinline__ uint32_t lds_pad(uint32_t i) { return i + (i >> 4); }
@@ -292,13 +292,8 @@ struct TwiddleLayout {
   static constexpr int total() { return offset(S::NPASS16); }
 };
 
-// Twiddles of one radix-16 pass for butterfly j = t (one butterfly per
-// thread): w[r-1] = exp(+2 pi i r (t mod NS) / (16 NS)), r = 1..15.  Issued
-// ahead of the barrier that precedes the pass, so their latency hides there.
-template <int N, int NS>
-__device__ __forceinline__ void load_twiddles16(cf *w, int t, const cf *tw) {
-  const cf *p = tw + (t % NS);
-  const cf w1 = p[0], w4 = p[NS];
+// w[r-1] = w^r, r = 1 ... 15, from w^1 and w^4.
+__device__ __forceinline__ void power_twiddles(cf *w, cf w1, cf w4) {
   const cf w2 = cmul(w1, w1), w8 = cmul(w4, w4);
   w[0] = w1;
   w[1] = w2;
@@ -310,6 +305,15 @@ __device__ __forceinline__ void load_twiddles16(cf *w, int t, const cf *tw) {
   w[6] = cmul(w[2], w4);
 #pragma unroll
   for (int r = 9; r < 16; r++) w[r - 1] = cmul(w[r - 9], w8);
+}
+
+// Twiddles of one radix-16 pass for butterfly j = t (one butterfly per
+// thread): w[r-1] = exp(+2 pi i r (t mod NS) / (16 NS)), r = 1..15.  Issued
+// ahead of the barrier that precedes the pass, so their latency hides there.
+template <int N, int NS>
+__device__ __forceinline__ void load_twiddles16(cf *w, int t, const cf *tw) {
+  const cf *p = tw + (t % NS);
+  power_twiddles(w, p[0], p[NS]);
 }
 
 // One Stockham pass of radix R: butterflies j = t + q*TPT (q < 16/R) read

@@ -37,13 +37,13 @@ int launch_mode(Ctx *c, const FlatArgs &a, dim3 grid, size_t lds) {
   return hip_ok(hipGetLastError(), "flat_kernel launch") ? 0 : -1;
 }
 
-// The kernel arguments of a launch over bins [bin0, bin0 + nb) of r (the
-// lag window [ws, we) of those bins; nb_total bins per output row).
-template <int N>
-int fill_args(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, size_t bin0, size_t nb, FlatArgs &a) {
+}  // namespace
+
+int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, size_t nb_total, size_t bin0, size_t nb,
+                   FlatArgs &a) {
   a.data = r.data;
   a.tmpl = r.tmpl;
-  a.twiddle = c->twiddles(N);
+  a.twiddle = c->twiddles(n);
   if (!a.twiddle) return -1;
   a.data_stride = r.data_stride;
   a.tmpl_stride = r.tmpl_stride;
@@ -74,11 +74,13 @@ int fill_args(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, s
   return 0;
 }
 
+namespace {
+
 template <int N>
 int launch_n(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, size_t bin0, size_t nb) {
   using S = FlatShape<N>;
   FlatArgs a;
-  if (fill_args<N>(c, r, ws, we, nb_total, bin0, nb, a) < 0) return -1;
+  if (flat_base_args(c, N, r, ws, we, nb_total, bin0, nb, a) < 0) return -1;
   const bool list = r.list != nullptr;
   const int dpw = a.dpw;
   dim3 grid;
@@ -168,6 +170,8 @@ size_t flat_twiddle_count(size_t n) {
     case 4096: return TwiddleLayout<4096>::total();
     case 8192: return TwiddleLayout<8192>::total();
     case 16384: return TwiddleLayout<16384>::total();
+    case 32768: return TwiddleLayout<32768>::total();
+    case 65536: return TwiddleLayout<65536>::total();
     default: return 0;
   }
 }
@@ -183,6 +187,8 @@ int flat_fill_twiddles(Ctx *c, size_t n, cf *tw) {
     case 4096: return fill_twiddles<4096>(c, tw);
     case 8192: return fill_twiddles<8192>(c, tw);
     case 16384: return fill_twiddles<16384>(c, tw);
+    case 32768: return fill_twiddles<32768>(c, tw);
+    case 65536: return fill_twiddles<65536>(c, tw);
     default: return fail("transform length %zu is not supported", n);
   }
 }
@@ -194,7 +200,7 @@ int flat_fill_args(Ctx *c, size_t n, const FlatRun &r, FlatArgs &a) {
   if (r.ws >= we) return fail("empty window (%zu, %zu)", r.ws, r.we);
   const size_t nb = (we - r.ws + r.binsize - 1) / r.binsize;
   if (nb > flat_max_bins<4096>()) return fail("too many bins for one launch (%zu)", nb);
-  return fill_args<4096>(c, r, r.ws, we, nb, 0, nb, a);
+  return flat_base_args(c, 4096, r, r.ws, we, nb, 0, nb, a);
 }
 
 bool flat_supported(size_t n) {
@@ -214,6 +220,9 @@ int launch_flat(Ctx *c, size_t n, const FlatRun &r) {
   FlatRun q = r;
   q.we = we;
   hipSetDevice(c->dev);
+  // a list may take either path from one call to the next (wide_takes)
+  if (r.list && r.hint && !c->capturing && !c->no_alloc && wide_reserve(c, n, q) < 0) return -1;
+  if (wide_takes(c, n, q)) return launch_wide(c, n, q);
   switch (n) {
     case 64: return launch_len<64>(c, q);
     case 128: return launch_len<128>(c, q);

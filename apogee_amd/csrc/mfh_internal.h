@@ -58,9 +58,10 @@ struct Ctx {
   cf *coarse_ctm = nullptr;
   int *coarse_sexp = nullptr;
   bool coarse_roots_ready = false;
-  // four-step lengths (32768, 65536): roots built, scratch budget per chunk
+  // two-kernel lengths (n >= 32768): roots built, scratch budget per chunk
   bool big_roots_ready[16] = {};  // by log2 of the column length
   long long big_chunk_bytes = 128ll << 20;  // measured best on gfx950 (256: +7%, 64: +16%)
+  int wide = 0;  // n = 8192 ... 65536 through launch_wide: 0 by the pair count, 1 always, 2 never
   int refine_grid_cap = 2048;  // workgroups of a list-driven (refine) launch, at most
   // pinned host word holding the last hierarchical refine's survivor count,
   // written by that launch (a sizing hint only: results never depend on it)
@@ -185,7 +186,17 @@ int launch_flat(Ctx *c, size_t n, const FlatRun &r);
 // window in one bin table), for kernels that run its per-pair path.
 struct FlatArgs;
 int flat_fill_args(Ctx *c, size_t n, const FlatRun &r, FlatArgs &a);
-// The two-kernel four-step flat filter for n = 32768 and 65536.
+// The kernel arguments of a launch over bins [bin0, bin0 + nb) of r (the lag
+// window [ws, we) of those bins; nb_total bins per output row).
+int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, size_t nb_total, size_t bin0, size_t nb,
+                   FlatArgs &a);
+// One workgroup per pair (or half of one) for n = 8192 ... 65536: whether a run
+// takes this path, the launch, and its buffers made in advance (for a
+// captured or allocation-free call of a list that may take either path).
+bool wide_takes(const Ctx *c, size_t n, const FlatRun &r);
+int launch_wide(Ctx *c, size_t n, const FlatRun &r);
+int wide_reserve(Ctx *c, size_t n, const FlatRun &r);
+// The two-kernel flat filter for n >= 32768.
 int launch_big(Ctx *c, size_t n, const FlatRun &r);
 // Four-step root tables for n = n1 * 256: w_n1^h (h < n1) then w_n^l (l < 256),
 // FP64-generated once per context.

@@ -11,12 +11,8 @@
 // the counter passes the tile count, so each workgroup reaches the exit.  One
 // workgroup of 1024 lanes per CU.
 //
-// Four-step lengths (32768, 65536) need a round trip through scratch between
-// their column and row transforms; inside one resident workgroup that round
-// trip is exposed latency (measured: time per pair independent of how many
-// workgroups share the device).  Their pairs therefore go, as a device list
-// with per-pair pool and output offsets, to the two-kernel four-step path of
-// the flat filter (columns of 16 lags per workgroup, then rows), queued just
+// Longer pairs (n >= 32768) go, as a device list with per-pair pool and output
+// offsets, to the flat filter's own launches for those lengths, queued just
 // before the persistent launch in the same stream and graph.
 //
 // Arithmetic.  Every pair runs the same product, transforms, twiddle tables
@@ -232,8 +228,8 @@ struct Queue {
   int ntiles = 0;
   long long nout = 0;
   long long npairs = 0;
-  // four-step pairs, grouped by (length, binsize, threshold, window): each
-  // group is one list-mode launch of the two-kernel path
+  // long pairs, grouped by (length, binsize, threshold, window): each group is
+  // one list-mode run of the flat filter
   struct BigGroup {
     int n;
     long long binsize;
@@ -341,7 +337,7 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     q->req_nc[r] = ncand[r];
     if (out_off) out_off[r] = nout;
     if (lg >= 15) {
-      // four-step: one list entry per pair, grouped by launch parameters
+      // long: one list entry per pair, grouped by launch parameters
       if (data_off[r] > INT32_MAX || tmpl_off[r] + (long long)ncand[r] * len > INT32_MAX)
         return fail("request %d: four-step spectra must start below pool element 2^31", r);
       size_t g = 0;
@@ -444,7 +440,7 @@ static int queue_launch(Queue *q, int64_t *idx, cf *val) {
   int *counter = (int *)c->scratch("q_counter", sizeof(int));
   if (!counter) return -1;
   if (c->prof_on && !c->capturing) q->prof_runs++;
-  // four-step pairs first: list-mode launches of the two-kernel path
+  // long pairs first: list-mode runs of the flat filter
   const int2 *blist = (const int2 *)c->bufs["q_big_list"].p;
   const long long *booff = (const long long *)c->bufs["q_big_ooff"].p;
   const int *bcount = (const int *)c->bufs["q_big_count"].p;
@@ -468,7 +464,7 @@ static int queue_launch(Queue *q, int64_t *idx, cf *val) {
     r.list_ooff = booff + G.first;
     r.list_cap = G.count;
     r.list_prof_name = "queue_big";
-    if (launch_big(c, (size_t)G.n, r) < 0) return -1;
+    if (launch_flat(c, (size_t)G.n, r) < 0) return -1;
   }
   QArgs a{};
   a.pool = q->pool;
