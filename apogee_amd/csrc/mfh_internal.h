@@ -194,6 +194,7 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
 // takes this path, the launch, and its buffers made in advance (for a
 // captured or allocation-free call of a list that may take either path).
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r);
+long long wide_min_pairs(size_t n);  // pairs from which an automatic run takes it
 int launch_wide(Ctx *c, size_t n, const FlatRun &r);
 int wide_reserve(Ctx *c, size_t n, const FlatRun &r);
 // The two-kernel flat filter for n >= 32768.

@@ -11,9 +11,12 @@
 // the counter passes the tile count, so each workgroup reaches the exit.  One
 // workgroup of 1024 lanes per CU.
 //
-// Longer pairs (n >= 32768) go, as a device list with per-pair pool and output
-// offsets, to the flat filter's own launches for those lengths, queued just
-// before the persistent launch in the same stream and graph.
+// Longer pairs go, as a device list with per-pair pool and output offsets, to
+// the flat filter's own launches for those lengths, queued just before the
+// persistent launch in the same stream and graph: n >= 32768 always, 8192 and
+// 16384 where a group of equal (n, binsize, threshold, window) has enough pairs
+// for the one-workgroup path (its 32 points per thread and two workgroups per
+// CU against one 1024-lane workgroup here).
 //
 // Arithmetic.  Every pair runs the same product, transforms, twiddle tables
 // and exact key rule as the per-request flat filter, so indices and values
@@ -43,6 +46,21 @@ struct QItem {
   float seed, inv_bs;             // threshold^2 (FP32) or 0; 1 / binsize
   int bshift, pad;                // log2(binsize) for powers of two, else -1
 };
+
+// An item of this request but for its template and output.
+QItem q_item(long long binsize, float thr, long long ws, long long we, long long d_off) {
+  QItem it{};
+  it.d_off = d_off;
+  it.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
+  it.binsize = (uint32_t)binsize;
+  const bool pow2 = (binsize & (binsize - 1)) == 0;
+  it.bshift = pow2 ? ilog2((int)binsize) : -1;
+  it.inv_bs = 1.0f / (float)binsize;
+  it.ws = (uint32_t)ws;
+  it.we = (uint32_t)we;
+  it.nb = (uint32_t)((we - ws + binsize - 1) / binsize);
+  return it;
+}
 
 struct QTile {
   int log2n, first, count, pad;  // length class, first item, items (<= slots)
@@ -336,9 +354,10 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     q->req_nb[r] = (int)nb;
     q->req_nc[r] = ncand[r];
     if (out_off) out_off[r] = nout;
-    if (lg >= 15) {
+    const bool far = data_off[r] > INT32_MAX || tmpl_off[r] + (long long)ncand[r] * len > INT32_MAX;
+    if (lg >= 15 || (lg >= 13 && !far)) {
       // long: one list entry per pair, grouped by launch parameters
-      if (data_off[r] > INT32_MAX || tmpl_off[r] + (long long)ncand[r] * len > INT32_MAX)
+      if (far)
         return fail("request %d: four-step spectra must start below pool element 2^31", r);
       size_t g = 0;
       for (; g < bigs.size(); g++) {
@@ -355,16 +374,7 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
         big_pairs[g].push_back({int2{(int)data_off[r], (int)(tmpl_off[r] + (long long)j * len)},
                                 nout + (long long)j * nb});
     } else {
-      QItem base{};
-      base.d_off = data_off[r];
-      base.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
-      base.binsize = (uint32_t)binsize[r];
-      const bool pow2 = (binsize[r] & (binsize[r] - 1)) == 0;
-      base.bshift = pow2 ? ilog2((int)binsize[r]) : -1;
-      base.inv_bs = 1.0f / (float)binsize[r];
-      base.ws = (uint32_t)ws[r];
-      base.we = (uint32_t)we[r];
-      base.nb = (uint32_t)nb;
+      const QItem base = q_item(binsize[r], thr, ws[r], we[r], data_off[r]);
       for (int j = 0; j < ncand[r]; j++) {
         QItem it = base;
         it.t_off = tmpl_off[r] + (long long)j * len;
@@ -374,6 +384,22 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     }
     nout += (long long)ncand[r] * nb;
     npairs += ncand[r];
+  }
+  // groups of 8192 and 16384 too small for the one-workgroup path
+  for (size_t g = 0; g < bigs.size();) {
+    const auto G = bigs[g];
+    if (ilog2(G.n) > kQMaxLog2 || (long long)big_pairs[g].size() >= wide_min_pairs((size_t)G.n)) {
+      g++;
+      continue;
+    }
+    for (auto &e : big_pairs[g]) {
+      QItem it = q_item(G.binsize, G.threshold, G.ws, G.we, e.first.x);
+      it.t_off = e.first.y;
+      it.o_off = e.second;
+      by_class[ilog2(G.n)].push_back(it);
+    }
+    bigs.erase(bigs.begin() + (long)g);
+    big_pairs.erase(big_pairs.begin() + (long)g);
   }
   std::vector<QItem> items;
   std::vector<QTile> tiles;

@@ -720,6 +720,8 @@ int wide_ready(Ctx *c, const FlatRun &r) {
 
 }  // namespace
 
+long long wide_min_pairs(size_t n) { return kWideMinPairs[ilog2((int)n) - 13]; }
+
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   if (n < 8192 || n > 65536 || c->wide == 2) return false;
   if (c->wide == 1) return true;
@@ -729,7 +731,7 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   // it takes, so it goes by the list's capacity
   if (r.list && r.hint && !c->capturing && !c->no_alloc)
     pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
-  return pairs >= kWideMinPairs[ilog2((int)n) - 13];
+  return pairs >= wide_min_pairs(n);
 }
 
 int launch_wide(Ctx *c, size_t n, const FlatRun &r) {

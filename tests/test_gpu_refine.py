@@ -199,3 +199,18 @@ def test_plan_errors_leave_the_queue_usable(gpu_device):
     q.plan(pool, n=[1024], data_offset=[0], template_offset=[1024], candidates=[3])
     out = q.run()
     assert out[0].shape == (3, 1) and good[0].shape == (2, 1)
+
+
+@pytest.mark.parametrize("n,c", [(8192, 300), (16384, 260), (8192, 20)])
+def test_long_groups_on_either_side_of_the_list_path(n, c, gpu_device):
+    """Groups of 8192 and 16384 large enough for the flat filter's list launches
+    and too small for them, beside other lengths and a second group."""
+    rng = np.random.default_rng(n + c)
+    reqs = [(cnoise(rng, n), cnoise(rng, (c, n)), n // 8, 0.0, None),
+            (cnoise(rng, 1024), cnoise(rng, (3, 1024)), 100, 0.0, None),
+            (cnoise(rng, n), cnoise(rng, (2, n)), 999, 300.0, (5, n - 3)),
+            (cnoise(rng, 32768), cnoise(rng, (1, 32768)), 32768, 0.0, None)]
+    q = mf.RefineQueue()
+    stage(q, reqs)
+    for _ in range(3):      # eager, captured, replayed
+        check_against_per_request(reqs, q.run(), gpu_device, "long groups")
