@@ -86,7 +86,7 @@ void *Ctx::host_stage(size_t bytes) {
   return stage;
 }
 
-bool peak_buffer(Ctx *c, size_t cells, PeakBuf &b) {
+bool peak_buffer(Ctx *c, size_t cells, PeakOut &b) {
   char *p = (char *)c->scratch("out_peaks", cells * (sizeof(int64_t) + sizeof(cf)));
   if (!p) return false;
   b.idx = (int64_t *)p;
@@ -156,27 +156,29 @@ bool host_block(const void *p, size_t bytes) {
   return a - it->first + bytes <= it->second;
 }
 
-long read_peaks(Ctx *c, const PeakBuf &b, size_t cells, size_t nb, int64_t *idx, void *val_c64, int32_t *counts,
+bool host_results(size_t cells, int64_t *idx, void *val_c64, void *rec, PeakOut &out) {
+  if (!cells) return false;
+  if (rec) {
+    if (!host_block(rec, cells * 16)) return false;
+    out.rec = (int4 *)rec;
+    return true;
+  }
+  if (!idx || (char *)val_c64 != (char *)idx + cells * sizeof(int64_t) ||
+      !host_block(idx, cells * (sizeof(int64_t) + sizeof(cf))))
+    return false;
+  out = peak_arrays(idx, val_c64);
+  return true;
+}
+
+long wait_peaks(Ctx *c, size_t cells, size_t nb, const int64_t *idx, int32_t *counts, const void *rec) {
+  if (!hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return -1;
+  return rec ? count_set(reinterpret_cast<const int64_t *>(rec), 2, cells, nb, counts)
+             : count_set(idx, 1, cells, nb, counts);
+}
+
+long read_peaks(Ctx *c, const PeakOut &b, size_t cells, size_t nb, int64_t *idx, void *val_c64, int32_t *counts,
                 void *rec) {
   const size_t bi = cells * sizeof(int64_t), bytes = bi + cells * sizeof(cf);
-  if (rec && cells && host_block(rec, cells * 16)) {
-    // the records go straight into the caller's page-locked buffer
-    hipLaunchKernelGGL(results_to_host, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, c->stream, b.idx,
-                       b.val, (long long)cells, 1, (char *)rec);
-    if (!hip_ok(hipGetLastError(), "results_to_host") ||
-        !hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))
-      return -1;
-    return count_set(reinterpret_cast<const int64_t *>(rec), 2, cells, nb, counts);
-  }
-  if (!rec && cells && idx && (char *)val_c64 == (char *)idx + bi && host_block(idx, bytes)) {
-    // [indices | values] straight into the caller's page-locked buffer
-    hipLaunchKernelGGL(results_to_host, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, c->stream, b.idx,
-                       b.val, (long long)cells, 0, (char *)idx);
-    if (!hip_ok(hipGetLastError(), "results_to_host") ||
-        !hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))
-      return -1;
-    return count_set(idx, 1, cells, nb, counts);
-  }
   char *st = (char *)c->host_stage(bytes);
   std::vector<char> pageable;
   const bool staged = st != nullptr;  // the readback kernel fills the staging in the caller's layout
@@ -538,10 +540,8 @@ extern "C" size_t mfh_nbins(size_t n, size_t binsize, size_t ws, size_t we) {
   return (we - ws + binsize - 1) / binsize;
 }
 
-extern "C" int mfh_flat_peaks_async(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t binsize, float threshold,
-                                    size_t ws, size_t we, int64_t *dev_idx, void *dev_val_c64) {
-  if (!ctx) return fail("null context");
-  Ctx *c = reinterpret_cast<Ctx *>(ctx);
+static int flat_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
+                    const mfh::PeakOut &out) {
   mfh::FlatRun r;
   r.data = c->data + (size_t)d0 * c->n;
   r.tmpl = c->tmpl + (size_t)t0 * c->n;
@@ -555,9 +555,15 @@ extern "C" int mfh_flat_peaks_async(mfh_ctx *ctx, int d0, int nd, int t0, int nt
   r.threshold = threshold;
   r.ws = ws;
   r.we = we;
-  r.out_idx = dev_idx;
-  r.out_val = (cf *)dev_val_c64;
+  r.out = out;
   return mfh::launch_flat(c, c->n, r);
+}
+
+extern "C" int mfh_flat_peaks_async(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t binsize, float threshold,
+                                    size_t ws, size_t we, int64_t *dev_idx, void *dev_val_c64) {
+  if (!ctx) return fail("null context");
+  return flat_run(reinterpret_cast<Ctx *>(ctx), d0, nd, t0, nt, binsize, threshold, ws, we,
+                  mfh::peak_arrays(dev_idx, dev_val_c64));
 }
 
 static long flat_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws,
@@ -570,20 +576,15 @@ static long flat_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t
   if (nb == 0) return fail("empty window (%zu, %zu)", ws, we);
   const size_t cells = (size_t)nd * (size_t)nt * nb;
   hipSetDevice(c->dev);
-  if (!rec && cells && (char *)val_c64 == (char *)idx + cells * sizeof(int64_t) &&
-      mfh::host_block(idx, cells * (sizeof(int64_t) + sizeof(cf)))) {
-    // [indices | values] in one page-locked mfh_host_alloc buffer: the
-    // filter writes the caller's arrays itself, with no readback step
-    if (mfh_flat_peaks_async(ctx, d0, nd, t0, nt, binsize, threshold, ws, we, idx, val_c64) < 0 ||
-        !hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))
-      return -1;
-    c->prof_collect();
-    return mfh::count_set(idx, 1, cells, nb, counts);
+  mfh::PeakOut out;
+  const bool direct = mfh::host_results(cells, idx, val_c64, rec, out);
+  if (!direct && !mfh::peak_buffer(c, cells, out)) return -1;
+  if (flat_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, out) < 0) {
+    hipStreamSynchronize(c->stream);  // a launch before the failure may still write the caller's buffer
+    return -1;
   }
-  mfh::PeakBuf pb;
-  if (!mfh::peak_buffer(c, cells, pb)) return -1;
-  if (mfh_flat_peaks_async(ctx, d0, nd, t0, nt, binsize, threshold, ws, we, pb.idx, pb.val) < 0) return -1;
-  const long total = mfh::read_peaks(c, pb, cells, nb, idx, val_c64, counts, rec);
+  const long total = direct ? mfh::wait_peaks(c, cells, nb, idx, counts, rec)
+                            : mfh::read_peaks(c, out, cells, nb, idx, val_c64, counts, rec);
   c->prof_collect();
   return total;
 }

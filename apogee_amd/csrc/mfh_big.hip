@@ -62,8 +62,7 @@ struct BigArgs {
   int nsplit;               // rows workgroups per pair (gridDim.y of the rows kernel)
   uint64_t *pkey;           // nsplit > 1: per-part bin tables [pair][part][nb]
   cf *pval;
-  int64_t *out_idx;
-  cf *out_val;
+  PeakOut out;
   uint32_t ws, we, binsize, nb, ostride;
   int bshift;
   float inv_bs, seed;
@@ -111,8 +110,8 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
     best = key > best ? key : best;
   }
   const long long o = a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-  a.out_idx[o + b] = best ? (int64_t)(~(uint32_t)(best & 0xffffffffull)) : -1;
-  a.out_val[o + b] = best ? a.pval[(pl * a.nsplit + bw) * (long long)nb + b] : cf{0.f, 0.f};
+  if (best) a.out.put(o + b, (long long)(~(uint32_t)best), a.pval[(pl * a.nsplit + bw) * (long long)nb + b]);
+  else a.out.none(o + b);
 }
 
 // Columns: 16 columns f1 of one pair per workgroup; lane = 16 * t + s, so the
@@ -321,17 +320,10 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     return;
   }
   const long long o = a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-  int64_t *oidx = a.out_idx + o;
-  cf *oval = a.out_val + o;
   for (int b = threadIdx.x; b < nb; b += 256) {
     const uint64_t key = bkey[b];
-    if (key) {
-      oidx[b] = (int64_t)(~(uint32_t)(key & 0xffffffffull));
-      oval[b] = bval[b];
-    } else {
-      oidx[b] = -1;
-      oval[b] = cf{0.f, 0.f};
-    }
+    if (key) a.out.put(o + b, (long long)(~(uint32_t)key), bval[b]);
+    else a.out.none(o + b);
   }
 }
 
@@ -447,8 +439,7 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
       a.we = (uint32_t)std::min(r.we, r.ws + (b0 + cnt) * r.binsize);
       a.nb = (uint32_t)cnt;
       a.ostride = (uint32_t)nb_total;
-      a.out_idx = r.out_idx + b0;
-      a.out_val = r.out_val + b0;
+      a.out = r.out.at(b0);
       const size_t lds = (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf) + cnt * (sizeof(uint64_t) + sizeof(cf));
       const long long row_blocks = np * nsplit;
       hipLaunchKernelGGL(big_rows_kernel<B>, dim3((unsigned)(row_blocks + fin_blocks)), dim3(256), lds, c->stream, a,

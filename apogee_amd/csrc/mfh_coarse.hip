@@ -526,18 +526,12 @@ __global__ void __launch_bounds__(256) coarse_mfma_kernel(const cf *data, long l
     const long long o = ((long long)(d0 + k) * nt + t0) * g.nb;
     if (g.nb == 1) {
       // one bin per pair (tpw <= 64): lane j writes template t0 + j
-      if (lane < cnt && !((f >> lane) & 1ull)) {
-        g.idx[o + lane] = -1;
-        g.val[o + lane] = cf{0.f, 0.f};
-      }
+      if (lane < cnt && !((f >> lane) & 1ull)) g.out.none(o + lane);
       continue;
     }
     for (int e = lane; e < cnt * g.nb; e += 64) {
       const int j = e / g.nb;
-      if (!((f >> j) & 1ull)) {
-        g.idx[o + e] = -1;
-        g.val[o + e] = cf{0.f, 0.f};
-      }
+      if (!((f >> j) & 1ull)) g.out.none(o + e);
     }
   }
 }
@@ -594,10 +588,7 @@ coarse_refine_kernel(const cf *data, long long data_stride, const cf *ctm, const
     base += __popcll(f);
     // one bin per pair: lane j answers template t0 + j
     const long long o = (long long)(d0 + k) * nt + t0 + lane;
-    if (lane < cnt && !mine) {
-      g.idx[o] = -1;
-      g.val[o] = cf{0.f, 0.f};
-    }
+    if (lane < cnt && !mine) g.out.none(o);
   }
   __syncthreads();  // the list is complete and the screen's LDS no longer read
   const int ns = wg_n;

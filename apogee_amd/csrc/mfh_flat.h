@@ -26,6 +26,7 @@
 // writes index and value, so the value always belongs to the reported lag.
 #pragma once
 #include "mfh_dft.h"
+#include "mfh_peak.h"
 #include "mfh_wave.h"
 
 namespace mfh {
@@ -34,8 +35,7 @@ struct FlatArgs {
   const cf *data;      // [rows][N] natural-order spectra (already offset to the first run row)
   const cf *tmpl;      // [rows][N] (already offset to the first run template)
   const cf *twiddle;   // per-pass tables, TwiddleLayout<N>
-  int64_t *out_idx;    // [nd][nt][nb]
-  cf *out_val;         // [nd][nt][nb]
+  PeakOut out;         // [nd][nt][nb]
   long long data_stride, tmpl_stride;  // elements between rows
   int nd, nt;          // run extent
   int dpw;             // data rows per workgroup (tiled mode)
@@ -505,13 +505,9 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
           zy |= u == uw ? __float_as_uint(v[u].y) : 0u;
         }
         const cf z = {__uint_as_float(zx), __uint_as_float(zy)};
-        a.out_idx[o] = (int64_t)kwin;
-        a.out_val[o] = z;
+        a.out.put(o, (long long)kwin, z);
       }
-      if (t == 0 && win == 0ull) {
-        a.out_idx[o] = -1;
-        a.out_val[o] = cf{0.f, 0.f};
-      }
+      if (t == 0 && win == 0ull) a.out.none(o);
     }
   } else {
     // ---- several bins: per-thread runs, wave reductions, LDS max ----------
@@ -581,8 +577,6 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
     // ---- the owner of each winning lag writes it; empty bins get -1/0 ----
     if (valid) {
       const long long o = (LIST && a.list_ooff) ? a.list_ooff[dd + slot] : ((long long)d * a.nt + tt) * a.ostride;
-      int64_t *oidx = a.out_idx + o;
-      cf *oval = a.out_val + o;
 #pragma unroll
       for (int u = 0; u < 16; u++) {
         const uint32_t k = (uint32_t)(t + u * TPT);
@@ -590,18 +584,12 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
           const uint64_t key = make_key(v[u], k, a.seed);
           if (key) {
             const uint32_t b = bin_of(k, a);
-            if (bins[b] == key) {
-              oidx[b] = (int64_t)k;
-              oval[b] = v[u];
-            }
+            if (bins[b] == key) a.out.put(o + b, (long long)k, v[u]);
           }
         }
       }
       for (int b = t; b < nb; b += TPT) {
-        if (bins[b] == 0ull) {
-          oidx[b] = -1;
-          oval[b] = cf{0.f, 0.f};
-        }
+        if (bins[b] == 0ull) a.out.none(o + b);
       }
     }
   }

@@ -61,8 +61,7 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
   a.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
   // Output rows are [nd][nt][nb_total]; a window piece writes bins
   // [bin0, bin0 + nb) of each row.
-  a.out_idx = r.out_idx + bin0;
-  a.out_val = r.out_val + bin0;
+  a.out = r.out.at(bin0);
   a.list = r.list;
   a.list_count = r.list_count;
   a.list_ooff = r.list_ooff;

@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) coarse_template_kernel(const cf *tmpl, lo
 // One atomic per wave: lanes that fire take consecutive slots after the
 // wave's base, found from the ballot.
 __global__ void gate_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, float thr, int nb,
-                            int64_t *out_idx, cf *out_val, int2 *list, int *count, int *other) {
+                            PeakOut out, int2 *list, int *count, int *other) {
   const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p == 0) *other = 0;  // the next call's counter
   const bool inside = p < (long long)nd * nt;
@@ -91,10 +91,7 @@ __global__ void gate_kernel(const int64_t *cidx, const cf *cval, int nd, int nt,
     const int slot = base + __popcll(ballot & ((1ull << lane) - 1ull));
     list[slot] = int2{(int)(p / nt), (int)(p % nt)};
   } else {
-    for (int b = 0; b < nb; b++) {
-      out_idx[p * nb + b] = -1;
-      out_val[p * nb + b] = cf{0.f, 0.f};
-    }
+    for (int b = 0; b < nb; b++) out.none(p * nb + b);
   }
 }
 
@@ -135,10 +132,7 @@ gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, float th
     const unsigned long long ballot = __ballot(fire);
     if (fire) surv[__popcll(ballot & ((1ull << lane) - 1ull))] = int2{d, tt};
     if (inside && !fire) {
-      for (int b = 0; b < nb; b++) {
-        fa.out_idx[p * fa.ostride + b] = -1;
-        fa.out_val[p * fa.ostride + b] = cf{0.f, 0.f};
-      }
+      for (int b = 0; b < nb; b++) fa.out.none(p * fa.ostride + b);
     }
     if (lane == 0) ns_sh = __popcll(ballot);
   }
@@ -216,7 +210,7 @@ int *hier_counter(Ctx *c, int parity) {
 // The refine's launch description (everything but the list fields): the
 // run's data rows and templates, its window, bins and threshold, its outputs.
 static FlatRun refine_base(Ctx *c, const cf *drows, int t0, int nd, int nt, size_t binsize, float threshold,
-                           size_t ws, size_t we, int64_t *idx, cf *val) {
+                           size_t ws, size_t we, const PeakOut &out) {
   FlatRun rr;
   rr.data = drows;
   rr.tmpl = c->tmpl + (size_t)t0 * c->n;
@@ -228,8 +222,7 @@ static FlatRun refine_base(Ctx *c, const cf *drows, int t0, int nd, int nt, size
   rr.threshold = threshold;
   rr.ws = ws;
   rr.we = we;
-  rr.out_idx = idx;
-  rr.out_val = val;
+  rr.out = out;
   return rr;
 }
 
@@ -261,7 +254,7 @@ static int launch_gate_refine(Ctx *c, const int64_t *cidx, const cf *cval, int n
 }
 
 int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-             float coarse_thr, int64_t *idx, cf *val, int *count_out, const cf *data_rows, const HierScratch *hs) {
+             float coarse_thr, const PeakOut &out, int *count_out, const cf *data_rows, const HierScratch *hs) {
   if (c->coarse_band <= 0) return fail("no coarse band: call mfh_hier_set_band first");
   if (!(coarse_thr >= 0.f) || !std::isfinite(coarse_thr))
     return fail("coarse threshold must be finite and nonnegative");
@@ -314,8 +307,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
       g.thr2 = std::nextafter((float)(w * w), 0.f);
     }
     g.nb = (int)nb;
-    g.idx = idx;
-    g.val = val;
+    g.out = out;
     g.list = list;
     g.count = count;
     g.zero = other;
@@ -323,7 +315,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
       // one launch: each workgroup of the screen refines its own survivors
       // (the count still goes to this call's counter; no list, no second
       // launch)
-      const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, idx, val);
+      const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, out);
       if (launch_coarse_refine(c, drows, (long long)n, t0, nd, nt, (int)cs, (int)ce, c->coarse_prec == 2, g, rr) < 0)
         return -1;
       if (!c->capturing && !hs) c->hier_parity ^= 1;
@@ -347,8 +339,8 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
   cr.threshold = coarse_thr;
   cr.ws = cs;
   cr.we = ce;
-  cr.out_idx = cidx;
-  cr.out_val = cval;
+  cr.out.idx = cidx;
+  cr.out.val = cval;
   cr.prof_name = "coarse";
   cr.zero = count;  // the coarse launch clears the survivor counter
   if (!mfma) {
@@ -356,7 +348,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
     if (gate_refine_fits(c, n, nb, ws, we, binsize)) {
       // the gate and the refine in one launch; the screen above cleared this
       // call's counter, the launch clears the next call's
-      const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, idx, val);
+      const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, out);
       if (launch_gate_refine(c, cidx, cval, nd, nt, coarse_thr, count, other, rr) < 0) return -1;
       if (!c->capturing && !hs) c->hier_parity ^= 1;
       if (count_out &&
@@ -366,7 +358,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
     }
     Ctx::ProfScope ps(c, "gate");
     hipLaunchKernelGGL(gate_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, c->stream, cidx, cval, nd,
-                       nt, coarse_thr, (int)nb, idx, val, list, count, other);
+                       nt, coarse_thr, (int)nb, out, list, count, other);
     if (!hip_ok(hipGetLastError(), "gate_kernel")) return -1;
   }
   // the screen has cleared the other counter: the next call uses it (a
@@ -374,7 +366,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
   // leave the context's pair untouched)
   if (!c->capturing && !hs) c->hier_parity ^= 1;
 
-  FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, idx, val);
+  FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, out);
   rr.list = list;
   rr.list_count = count;
   rr.list_cap = (int)pairs;
@@ -486,8 +478,8 @@ extern "C" int mfh_hier_coarse_max(mfh_ctx *ctx, int d0, int nd, int t0, int nt,
   cr.threshold = 0.f;
   cr.ws = cs;
   cr.we = ce;
-  cr.out_idx = cidx;
-  cr.out_val = cval;
+  cr.out.idx = cidx;
+  cr.out.val = cval;
   cr.prof_name = "coarse";
   std::vector<mfh::cf> v(pairs);
   if (mfh::launch_flat(c, m, cr) < 0 ||
@@ -515,13 +507,13 @@ static long long dbits(double x) {
 // launch parameters runs eagerly, the second identical call is captured into
 // a HIP graph, and later identical calls replay it with one launch.
 int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-                    float coarse_thr, int64_t *idx, cf *val, int *count_out) {
+                    float coarse_thr, const PeakOut &out, int *count_out) {
   if (!c->use_graphs || c->prof_on)
-    return hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, idx, val, count_out, nullptr);
+    return hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, count_out, nullptr);
   hipSetDevice(c->dev);
   if (c->coarse_band > 0 && hier_prepare(c) < 0) return -1;
   std::vector<long long> key = {d0, nd, t0, nt, (long long)binsize, fbits(threshold), (long long)ws, (long long)we,
-                                fbits(coarse_thr), (long long)(intptr_t)idx, (long long)(intptr_t)val,
+                                fbits(coarse_thr), (long long)(intptr_t)out.idx, (long long)(intptr_t)out.val, (long long)(intptr_t)out.rec,
                                 c->coarse_band, dbits(c->coarse_ref_f), c->coarse_prec, fbits(c->coarse_delta),
                                 c->refine_grid_cap, (long long)(intptr_t)c->coarse_tmpl, c->coarse_tpw, c->coarse_rpw, c->coarse_lds,
                                 c->coarse_fuse,
@@ -540,7 +532,7 @@ int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, floa
     if (!hip_ok(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
       return -1;
     c->capturing = true;
-    const int rc = hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, idx, val, nullptr, nullptr);
+    const int rc = hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, nullptr, nullptr);
     c->capturing = false;
     const bool ended = hip_ok(hipStreamEndCapture(c->stream, &g), "hipStreamEndCapture");
     if (rc < 0 || !ended) {
@@ -555,7 +547,7 @@ int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, floa
     if (!hip_ok(hipGraphLaunch(ex, c->stream), "hipGraphLaunch")) return -1;
     c->hier_parity ^= 1;
   } else {
-    if (hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, idx, val, nullptr, nullptr) < 0)
+    if (hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, nullptr, nullptr) < 0)
       return -1;
     c->last_key = key;
   }
@@ -575,8 +567,8 @@ extern "C" int mfh_hier_peaks_async(mfh_ctx *ctx, int d0, int nd, int t0, int nt
                                     int32_t *host_refined) {
   if (!ctx) return fail("null context");
   Ctx *c = reinterpret_cast<Ctx *>(ctx);
-  return mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, dev_idx,
-                              (mfh::cf *)dev_val_c64, host_refined);
+  return mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr,
+                              mfh::peak_arrays(dev_idx, dev_val_c64), host_refined);
 }
 
 static long hier_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws,
@@ -591,12 +583,16 @@ static long hier_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t
   if (nd < 1 || nt < 1) return fail("data/templates sub-range out of bounds");
   const size_t cells = (size_t)nd * (size_t)nt * nb;
   hipSetDevice(c->dev);
-  mfh::PeakBuf pb;
-  if (!mfh::peak_buffer(c, cells, pb)) return -1;
   int refined = 0;
-  if (mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, pb.idx, pb.val, &refined) < 0)
+  mfh::PeakOut out;
+  const bool direct = !c->use_graphs && mfh::host_results(cells, idx, val_c64, rec, out);
+  if (!direct && !mfh::peak_buffer(c, cells, out)) return -1;
+  if (mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, &refined) < 0) {
+    hipStreamSynchronize(c->stream);  // a launch before the failure may still write the caller's buffer
     return -1;
-  const long total = mfh::read_peaks(c, pb, cells, nb, idx, val_c64, counts, rec);
+  }
+  const long total = direct ? mfh::wait_peaks(c, cells, nb, idx, counts, rec)
+                            : mfh::read_peaks(c, out, cells, nb, idx, val_c64, counts, rec);
   if (total < 0) return -1;
   c->prof_collect();
   if (n_refined) *n_refined = refined;
@@ -675,8 +671,8 @@ extern "C" int mfh_hier_peaks_noalloc(mfh_ctx *ctx, int d0, int nd, int t0, int 
   hs.cval = (mfh::cf *)(base + kNoAllocHead + pairs * sizeof(int64_t));
   hs.list = (int2 *)(base + kNoAllocHead + pairs * (sizeof(int64_t) + sizeof(mfh::cf)));
   c->no_alloc = true;
-  const int rc = mfh::hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, dev_idx,
-                               (mfh::cf *)dev_val_c64, nullptr, nullptr, &hs);
+  const int rc = mfh::hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr,
+                               mfh::peak_arrays(dev_idx, dev_val_c64), nullptr, nullptr, &hs);
   c->no_alloc = false;
   return rc;
 }

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mfh_dft.h"
+#include "mfh_peak.h"
 
 namespace mfh {
 
@@ -132,23 +133,30 @@ struct Ctx {
   ~Ctx();
 };
 
+// Results in two arrays.
+inline PeakOut peak_arrays(int64_t *idx, void *val_c64) {
+  PeakOut o;
+  o.idx = idx;
+  o.val = (cf *)val_c64;
+  return o;
+}
 // A call's device results, laid out [cells indices | cells values] in the
 // context's "out_peaks" buffer so that one copy brings both back.
-struct PeakBuf {
-  int64_t *idx = nullptr;
-  cf *val = nullptr;
-};
-bool peak_buffer(Ctx *c, size_t cells, PeakBuf &b);
+bool peak_buffer(Ctx *c, size_t cells, PeakOut &b);
+// Whether the caller's results lie in an mfh_host_alloc buffer in a layout that
+// the filter kernels write themselves (records, or the values right after
+// the indices): then `out` is that buffer, and wait_peaks takes the place of
+// read_peaks.
+bool host_results(size_t cells, int64_t *idx, void *val_c64, void *rec, PeakOut &out);
+long wait_peaks(Ctx *c, size_t cells, size_t nb, const int64_t *idx, int32_t *counts, const void *rec);
 // Bring `cells` results to the caller's host arrays: a kernel queued on the
 // context's stream writes them in the caller's layout -- 16-byte {int64
 // index; complex64 value} records into `rec` (idx and val unused), else
-// [indices | values] -- straight into the caller's memory when it lies in an
-// mfh_host_alloc buffer (the values right after the indices, for idx/val),
-// else into the page-locked staging buffer followed by host copies (or
-// copy-engine transfers when no staging can be had); then waits for the
-// stream.  counts[p] (if set) = bins set of pair p, nb bins per pair.
-// Returns the total of set bins, or -1 (message set).
-long read_peaks(Ctx *c, const PeakBuf &b, size_t cells, size_t nb, int64_t *idx, void *val_c64, int32_t *counts,
+// [indices | values] -- into the page-locked staging buffer, followed by host
+// copies (or copy-engine transfers when no staging can be had); then waits
+// for the stream.  counts[p] (if set) = bins set of pair p, nb bins per pair.
+// Both return the total of set bins, or -1 (message set).
+long read_peaks(Ctx *c, const PeakOut &b, size_t cells, size_t nb, int64_t *idx, void *val_c64, int32_t *counts,
                 void *rec = nullptr);
 
 // One flat launch: pairs (data rows x template rows) from the given bases.
@@ -160,8 +168,7 @@ struct FlatRun {
   size_t binsize = 0;
   float threshold = 0.f;
   size_t ws = 0, we = 0;
-  int64_t *out_idx = nullptr;
-  cf *out_val = nullptr;
+  PeakOut out;
   // list mode: pairs (data row, template row) read from the device
   const int2 *list = nullptr;
   const int *list_count = nullptr;
@@ -225,8 +232,7 @@ int coarse_mfma_prepare(Ctx *c);
 struct CoarseGate {
   float thr2 = 0.f;
   int nb = 0;
-  int64_t *idx = nullptr;
-  cf *val = nullptr;
+  PeakOut out;
   int2 *list = nullptr;
   int *count = nullptr;
   int *zero = nullptr;  // set to 0 by the launch (the next call's counter)
@@ -255,7 +261,7 @@ struct HierScratch {
   int *spare = nullptr;
 };
 int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-             float coarse_thr, int64_t *idx, cf *val, int *count_out, const cf *data_rows,
+             float coarse_thr, const PeakOut &out, int *count_out, const cf *data_rows,
              const HierScratch *hs = nullptr);
 
 }  // namespace mfh

@@ -483,8 +483,7 @@ static int queue_launch(Queue *q, int64_t *idx, cf *val) {
     r.threshold = G.threshold;
     r.ws = (size_t)G.ws;
     r.we = (size_t)G.we;
-    r.out_idx = idx;
-    r.out_val = (cf *)val;
+    r.out = peak_arrays(idx, val);
     r.list = blist + G.first;
     r.list_count = bcount + g;
     r.list_ooff = booff + G.first;

@@ -220,10 +220,9 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
   hipSetDevice(c->dev);
   cf *spec = (cf *)c->scratch("series_spec", (size_t)nblocks * n * sizeof(cf));
   const size_t cells = (size_t)nblocks * nt * nb;
-  mfh::PeakBuf pb;
-  if (!spec || !mfh::peak_buffer(c, cells, pb)) return -1;
-  int64_t *didx = pb.idx;
-  cf *dval = pb.val;
+  mfh::PeakOut out;
+  const bool direct = mfh::host_results(cells, idx, val_c64, rec, out);
+  if (!spec || (!direct && !mfh::peak_buffer(c, cells, out))) return -1;
   const cf *dser;
   if (series_on_device) {
     dser = (const cf *)series_c64;
@@ -256,13 +255,12 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
     int g = 1;
     while (b0 + g < nblocks && win_start[b0 + g] == win_start[b0] && win_end[b0 + g] == win_end[b0]) g++;
     const size_t ws = win_start[b0], we = std::min(win_end[b0], n);
-    int64_t *oi = didx + (size_t)b0 * nt * nb;
-    cf *ov = dval + (size_t)b0 * nt * nb;
+    const mfh::PeakOut group = out.at((size_t)b0 * nt * nb);
     if (hier) {
       refined.push_back(0);
       // survivor counts are read from the device list counter per group
       int cnt = 0;
-      if (mfh::hier_run(c, 0, g, t0, nt, binsize, threshold, ws, we, coarse_thr, oi, ov, &cnt,
+      if (mfh::hier_run(c, 0, g, t0, nt, binsize, threshold, ws, we, coarse_thr, group, &cnt,
                         spec + (size_t)b0 * n) < 0 ||
           !hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))
         return -1;
@@ -279,13 +277,14 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
       r.threshold = threshold;
       r.ws = ws;
       r.we = we;
-      r.out_idx = oi;
-      r.out_val = ov;
+      r.out = group;
       if (mfh::launch_flat(c, n, r) < 0) return -1;
     }
     b0 += g;
   }
-  const long total = mfh::read_peaks(c, pb, cells, nb, idx, val_c64, counts, rec);  // waits for the stream
+  // both wait for the stream
+  const long total = direct ? mfh::wait_peaks(c, cells, nb, idx, counts, rec)
+                            : mfh::read_peaks(c, out, cells, nb, idx, val_c64, counts, rec);
   if (total < 0) return -1;
   wait_on_return.armed = false;
   c->prof_collect();

@@ -457,15 +457,19 @@ __device__ __forceinline__ void wide_select(const FlatArgs &a, const cf *v, uint
   sel.end();
 }
 
-// Write index (oidx null: keys are kept apart) and value of the bins whose
-// winning lag this wave holds.  Up to kWideLook bins, each lane looks at one
+// Write the peaks of the bins whose winning lag this wave holds, at o + bin of
+// the outputs (S = 1) or only their values, to pval (the keys go apart).  Up to kWideLook bins, each lane looks at one
 // bin's key and the wave then visits its own winners; past that the samples
 // are fewer than the bins, and the `hot` ones look up theirs.
 constexpr int kWideLook = 2048;
 template <class W, bool ONE>
 __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples &v, uint32_t hot, int t, int h,
-                                           int lane, int nb, const uint64_t *bins, int64_t *oidx, cf *oval) {
+                                           int lane, int nb, const uint64_t *bins, long long o, cf *pval) {
   constexpr int S = W::S, T = W::T;
+  auto put = [&](int b, uint32_t k, cf z) {
+    if constexpr (S == 1) a.out.put(o + b, (long long)k, z);
+    else pval[o + b] = z;
+  };
   if (ONE || nb <= kWideLook) {
     const int w0 = __builtin_amdgcn_readfirstlane(t);
 #pragma unroll 1
@@ -478,10 +482,7 @@ __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples 
         const int j = __builtin_ctzll(mine);
         const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)kwin, j);
         const cf z = v[(int)(k / S / T)];
-        if ((int)((k / S) % T) == t) {
-          if (oidx) oidx[b0 + j] = (int64_t)k;
-          oval[b0 + j] = z;
-        }
+        if ((int)((k / S) % T) == t) put(b0 + j, k, z);
       }
     }
   } else {
@@ -492,10 +493,7 @@ __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples 
       const uint32_t k = (uint32_t)(S * (t + u * T) + h);
       if (k - a.ws < a.we - a.ws) {
         const uint32_t b = bin_of(k, a);
-        if (k == ~(uint32_t)bins[b]) {  // an empty bin's key is 0: past every lag
-          if (oidx) oidx[b] = (int64_t)k;
-          oval[b] = z;
-        }
+        if (k == ~(uint32_t)bins[b]) put((int)b, k, z);  // an empty bin's key is 0: past every lag
       }
     }
   }
@@ -565,28 +563,12 @@ __global__ void __launch_bounds__(W::T) __attribute__((amdgpu_waves_per_eu(4))) 
     if (hot) wide_select<W, ONE, DENSE>(a, v, hot, t, h, bins);
     __syncthreads();
     long long o;
-    int64_t *oidx = nullptr;
-    uint64_t *okey = nullptr;
-    cf *oval;
-    if constexpr (S == 1) {
-      o = (LIST && a.list_ooff) ? a.list_ooff[wa.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-      oidx = a.out_idx + o;
-      oval = a.out_val + o;
-    } else {
-      o = unit * nb;
-      okey = wa.pkey + o;
-      oval = wa.pval + o;
-    }
-    if (hot) wide_write<W, ONE>(a, WideSamples(v), hot, t, h, lane, nb, bins, oidx, oval);
+    if constexpr (S > 1) o = unit * nb;
+    else o = (LIST && a.list_ooff) ? a.list_ooff[wa.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
+    if (hot) wide_write<W, ONE>(a, WideSamples(v), hot, t, h, lane, nb, bins, o, wa.pval);
     for (int b = threadIdx.x; b < nb; b += T) {
-      if constexpr (S == 1) {
-        if (bins[b] == 0ull) {
-          oidx[b] = -1;
-          oval[b] = cf{0.f, 0.f};
-        }
-      } else {
-        okey[b] = bins[b];
-      }
+      if constexpr (S > 1) wa.pkey[o + b] = bins[b];
+      else if (bins[b] == 0ull) a.out.none(o + b);
     }
     if constexpr (LIST) __syncthreads();  // the space is free for the next unit's exchange
     w += gridDim.x;
@@ -623,8 +605,8 @@ __global__ void __launch_bounds__(256) wide_finish_kernel(WideArgs wa) {
     best = key > best ? key : best;
   }
   const long long o = (LIST && a.list_ooff) ? a.list_ooff[wa.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-  a.out_idx[o + b] = best ? (int64_t)(~(uint32_t)best) : -1;
-  a.out_val[o + b] = best ? wa.pval[(pl * S + bw) * nb + b] : cf{0.f, 0.f};
+  if (best) a.out.put(o + b, (long long)(~(uint32_t)best), wa.pval[(pl * S + bw) * nb + b]);
+  else a.out.none(o + b);
 }
 
 template <class W>
