@@ -379,6 +379,18 @@ __device__ __forceinline__ void stockham_load(cf *v, int t, const cf *xch) {
   }
 }
 
+// Orders a slot's LDS stores before its later loads: a barrier, or for a slot
+// inside one wave only a compiler fence.
+template <bool WAVE>
+__device__ __forceinline__ void slot_sync() {
+  if constexpr (WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
 // Full inverse FFT of the slot's N points held in v; returns with thread t
 // holding z[t + u*TPT].  Each exchange is store -> barrier -> load, and the
 // barrier that protects the buffer from the next store sits just before that
@@ -390,10 +402,14 @@ __device__ __forceinline__ void stockham_load(cf *v, int t, const cf *xch) {
 // the thread only, so a kernel that runs many pairs per thread derives them
 // once instead of per pair.  The values, and so the results, are bit for bit
 // those of the per-pair derivation.
-template <int N, bool HOISTED = false>
+//
+// WAVE: the slot's threads are consecutive lanes of one wave (TPT <= 64), whose
+// LDS operations execute in order, so the exchanges need no barrier.
+template <int N, bool HOISTED = false, bool WAVE = false>
 __device__ __forceinline__ void inverse_fft(cf *v, int t, cf *xch, const cf *tw, const cf *wfirst = nullptr) {
   using S = FlatShape<N>;
   using L = TwiddleLayout<N>;
+  static_assert(!WAVE || S::TPT <= 64, "a wave's slot");
   constexpr int F = S::FIRST;
   constexpr int NS0 = L::NS0;
   cf w[15];
@@ -401,23 +417,23 @@ __device__ __forceinline__ void inverse_fft(cf *v, int t, cf *xch, const cf *tw,
     stockham_pass<N, F, 1>(v, w);
     stockham_store<N, F, 1>(v, t, xch);
     if constexpr (!HOISTED) load_twiddles16<N, NS0>(w, t, tw + L::offset(0));
-    __syncthreads();
+    slot_sync<WAVE>();
     stockham_load<N>(v, t, xch);
   }
   stockham_pass<N, 16, NS0>(v, (HOISTED && F > 1) ? wfirst : w);
   if constexpr (S::NPASS16 >= 2) {
-    if constexpr (F > 1) __syncthreads();
+    if constexpr (F > 1) slot_sync<WAVE>();
     stockham_store<N, 16, NS0>(v, t, xch);
     if constexpr (!(HOISTED && F == 1)) load_twiddles16<N, NS0 * 16>(w, t, tw + L::offset(1));
-    __syncthreads();
+    slot_sync<WAVE>();
     stockham_load<N>(v, t, xch);
     stockham_pass<N, 16, NS0 * 16>(v, (HOISTED && F == 1) ? wfirst : w);
   }
   if constexpr (S::NPASS16 >= 3) {
-    __syncthreads();
+    slot_sync<WAVE>();
     stockham_store<N, 16, NS0 * 16>(v, t, xch);
     load_twiddles16<N, NS0 * 256>(w, t, tw + L::offset(2));
-    __syncthreads();
+    slot_sync<WAVE>();
     stockham_load<N>(v, t, xch);
     stockham_pass<N, 16, NS0 * 256>(v, w);
   }
@@ -446,6 +462,45 @@ enum BinMode : int {
   kGeneral = 2,  // anything else
 };
 
+// One bin, slots of at most 64 lanes (n <= 1024): the slot's largest |z|^2
+// above the seed, lowest lag first, by lane exchanges alone -- the key that the
+// per-sample scan and the LDS maximum build, without the 64-bit LDS atomic
+// per lane that bounded these lengths -- as a record in LDS, which its owner (or
+// lane 0, where nothing beats the seed) leaves in `res`.
+template <int N>
+__device__ __forceinline__ void one_bin_in_wave(const FlatArgs &a, const cf *v, int t, int4 *res) {
+  constexpr int TPT = FlatShape<N>::TPT;
+  float mb[16];
+#pragma unroll
+  for (int u = 0; u < 16; u++) mb[u] = __builtin_fmaf(v[u].x, v[u].x, v[u].y * v[u].y);
+  if (a.ws != 0 || a.we != (uint32_t)N) {
+#pragma unroll
+    for (int u = 0; u < 16; u++) mb[u] = (uint32_t)(t + u * TPT) - a.ws < a.we - a.ws ? mb[u] : 0.f;
+  }
+  float m = 0.f;  // a NaN is never the larger operand of fmaxf
+#pragma unroll
+  for (int u = 0; u < 16; u++) m = fmaxf(m, mb[u]);
+  const uint32_t gm = group_umax<TPT>(__float_as_uint(m));  // nonnegative floats order like their bits
+  const bool hot = __uint_as_float(gm) > a.seed;
+  if (__ballot(hot)) {
+    int bu = -1;
+#pragma unroll
+    for (int u = 15; u >= 0; u--) bu = __float_as_uint(mb[u]) == gm ? u : bu;
+    const uint32_t mine = hot && bu >= 0 ? (uint32_t)(t + bu * TPT) : 0xffffffffu;
+    const uint32_t kwin = group_umin<TPT>(mine);
+    if (mine == kwin && mine != 0xffffffffu) {
+      uint32_t zx = 0u, zy = 0u;
+#pragma unroll
+      for (int u = 0; u < 16; u++) {
+        zx |= u == bu ? __float_as_uint(v[u].x) : 0u;
+        zy |= u == bu ? __float_as_uint(v[u].y) : 0u;
+      }
+      *res = int4{(int)kwin, 0, (int)zx, (int)zy};
+    }
+  }
+  if (!hot && t == 0) *res = int4{-1, -1, 0, 0};
+}
+
 // The end of one pair's work in the flat kernel, after its inverse FFT has
 // left z[t + u*TPT] in v: the per-bin keys of the lags in the window, the
 // workgroup's bin maxima in LDS, and the writes of each bin's winning lag and
@@ -463,11 +518,10 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
     // ---- one bin: a wave key, one LDS max; the winning lag's owner writes ----
     uint64_t wkey = 0ull;
     bool have = false;
-    if constexpr (TPT >= 64) {
-      if (a.ws == 0 && a.we == (uint32_t)N) have = one_bin_wave_key<TPT>(v, t, a.seed, wkey);
-      else if ((a.ws & 63u) == 0 && (a.we & 63u) == 0)
-        have = one_bin_wave_key<TPT, true>(v, t, a.seed, wkey, a.ws, a.we);
-    }
+    static_assert(TPT > 64, "shorter slots: one_bin_in_wave");
+    if (a.ws == 0 && a.we == (uint32_t)N) have = one_bin_wave_key<TPT>(v, t, a.seed, wkey);
+    else if ((a.ws & 63u) == 0 && (a.we & 63u) == 0)
+      have = one_bin_wave_key<TPT, true>(v, t, a.seed, wkey, a.ws, a.we);
     if (!have) {
       // per-sample scan: strict, so the lowest lag keeps a tie
       float bm = a.seed;
@@ -483,11 +537,9 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
       }
       const uint64_t key =
           bu >= 0 ? ((uint64_t)__float_as_uint(bm) << 32) | (uint64_t)(~(uint32_t)(t + bu * TPT)) : 0ull;
-      if constexpr (TPT >= 64) wkey = wave_max_u64(key);
-      else wkey = key;  // several slots per wave: every lane raises its own key
+      wkey = wave_max_u64(key);
     }
-    if (TPT >= 64 ? (lane == 0 && wkey) : wkey != 0ull)
-      atomicMax((unsigned long long *)&bins[0], (unsigned long long)wkey);
+    if (lane == 0 && wkey) atomicMax((unsigned long long *)&bins[0], (unsigned long long)wkey);
     __syncthreads();
     if (valid) {
       const long long o = (LIST && a.list_ooff) ? a.list_ooff[dd + slot] : ((long long)d * a.nt + tt) * a.ostride;
@@ -572,7 +624,7 @@ __device__ __forceinline__ void select_and_write(const FlatArgs &a, int nb, cons
       }
       if (acc) atomicMax((unsigned long long *)&bins[acc_bin], (unsigned long long)acc);
     }
-    __syncthreads();
+    slot_sync<(TPT <= 64)>();
 
     // ---- the owner of each winning lag writes it; empty bins get -1/0 ----
     if (valid) {
@@ -631,12 +683,18 @@ flat_kernel(FlatArgs a) {
     // survivors most of a refine grid leaves here, before any other load)
     if (dbeg >= dend) return;
   }
+  // one bin in slots of at most a wave: records meet in LDS, so that the
+  // workgroup's neighbouring results are stored by neighbouring lanes
+  constexpr bool SMALL = MODE == kOneBin && TPT <= 64;
+  int4 *res_all = reinterpret_cast<int4 *>(bins_all);
   // the first twiddled pass's twiddles, once for every pair this thread runs
   cf wfirst[15];
   first_twiddles<N>(wfirst, t0, a.twiddle);
   // both bin buffers start empty
-  for (int i = threadIdx.x; i < 2 * S::SLOTS * nb; i += S::WG) bins_all[i] = 0ull;
-  __syncthreads();
+  if constexpr (!SMALL) {
+    for (int i = threadIdx.x; i < 2 * S::SLOTS * nb; i += S::WG) bins_all[i] = 0ull;
+    __syncthreads();
+  }
 
   const int dstep = LIST ? (int)gridDim.x * S::SLOTS : 1;
   // list mode: each pair's list entry is read one trip ahead, so the load
@@ -691,8 +749,30 @@ flat_kernel(FlatArgs a) {
 #pragma unroll
       for (int u = 0; u < 16; u++) v[u] = cmul_conj(dv[u], tv[u]);
     }
-    inverse_fft<N, true>(v, t, xch, a.twiddle, wfirst);
-    select_and_write<N, MODE, LIST>(a, nb, v, t, lane, bins, bins_next, valid, d, tt, dd, slot);
+    inverse_fft<N, true, (TPT <= 64)>(v, t, xch, a.twiddle, wfirst);
+    if constexpr (SMALL) {
+      int4 *res = res_all + (it & 1) * S::SLOTS;  // the other half's last readers are past this pair's barrier
+      one_bin_in_wave<N>(a, v, t, res + slot);
+      __syncthreads();
+      if ((int)threadIdx.x < S::SLOTS) {
+        int d2 = d, t2 = (int)(blockIdx.x * S::SLOTS + threadIdx.x);
+        bool real = t2 < a.nt;
+        long long o;
+        if constexpr (LIST) {
+          const int li = dd + (int)threadIdx.x;
+          real = li < dend;
+          const int2 pr = real ? a.list[li] : int2{0, 0};
+          d2 = pr.x;
+          t2 = pr.y;
+          o = a.list_ooff && real ? a.list_ooff[li] : ((long long)d2 * a.nt + t2) * a.ostride;
+        } else {
+          o = ((long long)d2 * a.nt + t2) * a.ostride;
+        }
+        if (real) a.out.put_record(o, res[threadIdx.x]);
+      }
+    } else {
+      select_and_write<N, MODE, LIST>(a, nb, v, t, lane, bins, bins_next, valid, d, tt, dd, slot);
+    }
   }
 }
 

@@ -18,7 +18,9 @@ constexpr size_t kLdsLimit = 160 * 1024;
 template <int N>
 size_t flat_lds_bytes(size_t nb) {
   using S = FlatShape<N>;
-  return (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf) + 2 * (size_t)S::SLOTS * nb * sizeof(uint64_t);
+  // two tables of bin keys, or of records (16 bytes) for one bin at n <= 1024
+  const size_t cell = nb == 1 && S::TPT <= 64 ? sizeof(int4) : sizeof(uint64_t);
+  return (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf) + 2 * (size_t)S::SLOTS * nb * cell;
 }
 
 template <int N>

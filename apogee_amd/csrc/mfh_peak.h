@@ -20,6 +20,15 @@ struct PeakOut {
       val[o] = z;
     }
   }
+  // a record as put() stores it
+  __device__ __forceinline__ void put_record(long long o, int4 r) const {
+    if (rec) {
+      rec[o] = r;
+    } else {
+      idx[o] = (long long)(((unsigned long long)(unsigned)r.y << 32) | (unsigned)r.x);
+      val[o] = cf{__int_as_float(r.z), __int_as_float(r.w)};
+    }
+  }
   __device__ __forceinline__ void none(long long o) const { put(o, -1, cf{0.f, 0.f}); }
   PeakOut at(size_t o) const {
     PeakOut r;

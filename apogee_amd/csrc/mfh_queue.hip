@@ -163,7 +163,7 @@ __device__ __forceinline__ void q_flat(const QArgs &a, const QTile &tile, cf *sm
   cf v[16];
 #pragma unroll
   for (int u = 0; u < 16; u++) v[u] = cmul_conj(D[t + u * TPT], T[t + u * TPT]);
-  inverse_fft<N>(v, t, xch, a.tw[FlatShape<N>::LOGN]);
+  inverse_fft<N, false, (TPT <= 64)>(v, t, xch, a.tw[FlatShape<N>::LOGN]);
   __syncthreads();  // every slot's last exchange read is done
   uint64_t *bkey = reinterpret_cast<uint64_t *>(xch);
   const int nb = (int)it.nb;

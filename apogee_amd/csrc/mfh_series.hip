@@ -44,7 +44,7 @@ series_forward_kernel(const cf *series, long long nseries, const BlockStarts sta
     const cf x = (valid && k < nseries) ? series[k] : cf{0.f, 0.f};
     v[u] = cf{x.x * inv, -(x.y * inv)};
   }
-  inverse_fft<N>(v, t, xch_all + slot * S::XSTRIDE, tw);
+  inverse_fft<N, false, (TPT <= 64)>(v, t, xch_all + slot * S::XSTRIDE, tw);
   if (valid) {
     cf *o = out + (long long)b * N;
 #pragma unroll

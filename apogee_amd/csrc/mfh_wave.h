@@ -53,4 +53,35 @@ __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
   return row_readlanes_min(v);
 }
 
+// Extremum over groups of G consecutive lanes (G = 4 ... 64, aligned), every
+// lane receiving its group's: the first of wave_umax's steps, for half a wave
+// the exchange of neighbouring rows of 16.  Call with the whole wave active.
+template <int G>
+__device__ __forceinline__ uint32_t group_umax(uint32_t v) {
+  if constexpr (G == 64) return wave_umax(v);
+  v = dpp_umax<0xB1>(v);
+  v = dpp_umax<0x4E>(v);
+  if constexpr (G >= 8) v = dpp_umax<0x141>(v);
+  if constexpr (G >= 16) v = dpp_umax<0x140>(v);
+  if constexpr (G >= 32) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max(s[0], s[1]);
+  }
+  return v;
+}
+
+template <int G>
+__device__ __forceinline__ uint32_t group_umin(uint32_t v) {
+  if constexpr (G == 64) return wave_umin(v);
+  v = dpp_umin<0xB1>(v);
+  v = dpp_umin<0x4E>(v);
+  if constexpr (G >= 8) v = dpp_umin<0x141>(v);
+  if constexpr (G >= 16) v = dpp_umin<0x140>(v);
+  if constexpr (G >= 32) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = min(s[0], s[1]);
+  }
+  return v;
+}
+
 }  // namespace mfh
