@@ -416,6 +416,8 @@ class Context:
         self._h = ctypes.c_void_p(h)
         self.last_refinements = 0
         self._bound = {}
+        # nothing here reads the number of reported bins a run returns
+        self.set_tuning("totals", 0)
 
     # ------------------------------------------------------------ lifetime
     def destroy(self):

@@ -40,6 +40,7 @@ struct Ctx {
   // from then on, so the caller's buffer is never modified.
   int own_bank(bool templates);
   int tune_dpw = 0;          // 0: automatic
+  bool totals = true;        // calls with host results return how many bins are set
   // hierarchical state: coarse band, bank-wide reference fraction (< 0: per
   // template), scaled coarse templates [nt][band], rebuilt when dirty
   int coarse_band = 0;
@@ -155,7 +156,8 @@ long wait_peaks(Ctx *c, size_t cells, size_t nb, const int64_t *idx, int32_t *co
 // [indices | values] -- into the page-locked staging buffer, followed by host
 // copies (or copy-engine transfers when no staging can be had); then waits
 // for the stream.  counts[p] (if set) = bins set of pair p, nb bins per pair.
-// Both return the total of set bins, or -1 (message set).
+// Both return the total of set bins (0 uncounted when neither counts nor
+// Ctx::totals ask for it), or -1 (message set).
 long read_peaks(Ctx *c, const PeakOut &b, size_t cells, size_t nb, int64_t *idx, void *val_c64, int32_t *counts,
                 void *rec = nullptr);
 

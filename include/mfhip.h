@@ -348,7 +348,9 @@ long mfh_hier_run_series_rec(mfh_ctx *ctx, const void *series_c64, size_t nserie
  * survivors in the same launch), "big_chunk_mb" (scratch
  * per column / row launch pair at n >= 32768), "wide" (n = 8192 ... 65536, one
  * workgroup per pair or half of one: 0 = by the pair count, 1 = always,
- * 2 = never; results are the same), "graphs" (0/1: replay the
+ * 2 = never; results are the same), "totals" (1 by default; 0: runs with host
+ * results return 0 instead of the number of reported bins unless per-pair
+ * counts are asked for, which saves a pass over the results), "graphs" (0/1: replay the
  * hierarchical sequence from HIP graphs; off by default, measured slower).
  * Replaces: MF_MFTILE / MF_PBMAX environment knobs (src/matchfilt.c:93-107). */
 int mfh_set_tuning(mfh_ctx *ctx, const char *key, long value);
