@@ -43,6 +43,7 @@ struct FlatArgs {
   const int *list_count;  // list mode: number of pairs in the list
   const long long *list_ooff;  // list mode: output element offset per pair (null: row-major d*nt + t)
   uint32_t ws, we;     // lag window [ws, we)
+  const uint2 *win;    // tiled mode, if set: each data row's own window (as many bins each)
   uint32_t binsize, nb;  // nb: bins of this launch
   uint32_t ostride;      // output elements between pairs (>= nb)
   int bshift;          // log2(binsize) when a power of two, else -1
@@ -707,6 +708,12 @@ flat_kernel(FlatArgs a) {
     // cheaper than the registers the hoisted copies would pin.
     int t = t0;
     asm volatile("" : "+v"(t));
+    if constexpr (!LIST) {
+      if (a.win) {  // uniform: dd is the tile's row
+        a.ws = a.win[dd].x;
+        a.we = a.win[dd].y;
+      }
+    }
     uint64_t *bins = bins_all + ((it & 1) * S::SLOTS + slot) * nb;
     uint64_t *bins_next = bins_all + (((it + 1) & 1) * S::SLOTS + slot) * nb;
     int d = dd;

@@ -51,6 +51,7 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
   a.tmpl_stride = r.tmpl_stride;
   a.nd = r.nd;
   a.nt = r.nt;
+  a.win = r.win;
   a.ws = (uint32_t)ws;
   a.we = (uint32_t)we;
   a.binsize = (uint32_t)r.binsize;
@@ -104,7 +105,7 @@ int launch_n(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, si
   const size_t lds = flat_lds_bytes<N>(nb);
   int mode = kGeneral;
   if (nb == 1) mode = kOneBin;
-  else if (ws % 64 == 0 && (we % 64 == 0) && r.binsize % 64 == 0) mode = kAligned;
+  else if ((r.win ? r.win_aligned : ws % 64 == 0 && we % 64 == 0) && r.binsize % 64 == 0) mode = kAligned;
   Ctx::ProfScope ps(c, list ? r.list_prof_name : r.prof_name);
   if (list) {
     if (mode == kOneBin) return launch_mode<N, kOneBin, true>(c, a, grid, lds);
@@ -211,6 +212,22 @@ bool flat_supported(size_t n) {
       return true;
     default:
       return false;
+  }
+}
+
+size_t flat_row_window_bins(const Ctx *c, size_t n, const FlatRun &r) {
+  if (wide_takes(c, n, r)) return wide_table_bins(n);
+  switch (n) {
+    case 64: return flat_max_bins<64>();
+    case 128: return flat_max_bins<128>();
+    case 256: return flat_max_bins<256>();
+    case 512: return flat_max_bins<512>();
+    case 1024: return flat_max_bins<1024>();
+    case 2048: return flat_max_bins<2048>();
+    case 4096: return flat_max_bins<4096>();
+    case 8192: return flat_max_bins<8192>();
+    case 16384: return flat_max_bins<16384>();
+    default: return 0;
   }
 }
 

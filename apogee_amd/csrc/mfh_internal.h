@@ -170,6 +170,11 @@ struct FlatRun {
   size_t binsize = 0;
   float threshold = 0.f;
   size_t ws = 0, we = 0;
+  // Tiled mode, if set: a device table of each data row's own window, all with
+  // the bin count of [ws, we) and at most flat_row_window_bins() of them;
+  // win_aligned: every edge is a multiple of 64 lags.
+  const uint2 *win = nullptr;
+  bool win_aligned = false;
   PeakOut out;
   // list mode: pairs (data row, template row) read from the device
   const int2 *list = nullptr;
@@ -185,6 +190,9 @@ struct FlatRun {
 };
 
 bool flat_supported(size_t n);
+// The most bins a run with a window per data row may have (0: this length's path
+// takes one window per run).
+size_t flat_row_window_bins(const Ctx *c, size_t n, const FlatRun &r);
 // Per-pass twiddle table size (complex elements) and its FP64 generation.
 size_t flat_twiddle_count(size_t n);
 int flat_fill_twiddles(Ctx *c, size_t n, cf *tw);
@@ -203,6 +211,7 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
 // takes this path, the launch, and its buffers made in advance (for a
 // captured or allocation-free call of a list that may take either path).
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r);
+size_t wide_table_bins(size_t n);    // bins of one launch
 long long wide_min_pairs(size_t n);  // pairs from which an automatic run takes it
 int launch_wide(Ctx *c, size_t n, const FlatRun &r);
 int wide_reserve(Ctx *c, size_t n, const FlatRun &r);
@@ -213,11 +222,19 @@ int launch_big(Ctx *c, size_t n, const FlatRun &r);
 const cf *big_roots(Ctx *c, int n1);
 // Start offsets of run_series blocks as the forward kernels read them: up to
 // kInline in the kernel arguments themselves (no upload), else a device table.
+// With `win_out` set the forward also leaves the blocks' windows there, as the
+// filter behind it reads them: no upload or launch of their own.
 struct BlockStarts {
   static constexpr int kInline = 64;
   const long long *dev = nullptr;  // device table of every block, or null: `inl` holds them
+  uint2 *win_out = nullptr;
+  int nwin = 0;
   long long inl[kInline];
+  uint2 win[kInline];
   __device__ long long operator[](int b) const { return dev ? dev[b] : inl[b]; }
+  __device__ void store_windows() const {
+    if (win_out && blockIdx.x == 0 && blockIdx.y == 0 && (int)threadIdx.x < nwin) win_out[threadIdx.x] = win[threadIdx.x];
+  }
 };
 // Forward spectra of run_series blocks into out [nblocks][n] (device).
 int launch_series_forward(Ctx *c, const cf *series, size_t nseries, const BlockStarts &starts, int nblocks,

@@ -502,7 +502,7 @@ __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples 
 template <class W, bool ONE, bool DENSE, bool LIST>
 __global__ void __launch_bounds__(W::T) __attribute__((amdgpu_waves_per_eu(4))) wide_kernel(WideArgs wa) {
   constexpr int S = W::S, T = W::T, N = W::N;
-  const FlatArgs &a = wa.f;
+  FlatArgs &a = wa.f;
   extern __shared__ __align__(16) unsigned char smem[];
   float *x = reinterpret_cast<float *>(smem);
   uint64_t *bins = reinterpret_cast<uint64_t *>(smem);  // after the last exchange, in the same space
@@ -534,6 +534,12 @@ __global__ void __launch_bounds__(W::T) __attribute__((amdgpu_waves_per_eu(4))) 
     } else {
       tt = (int)((wa.p0 + pl) / a.nd);
       d = (int)((wa.p0 + pl) % a.nd);
+    }
+    if constexpr (!LIST) {
+      if (a.win) {
+        a.ws = a.win[d].x;
+        a.we = a.win[d].y;
+      }
     }
     int t = threadIdx.x;
     asm volatile("" : "+v"(t));
@@ -701,6 +707,16 @@ int wide_ready(Ctx *c, const FlatRun &r) {
 }
 
 }  // namespace
+
+size_t wide_table_bins(size_t n) {
+  switch (n) {
+    case 8192: return wide_max_bins<WideShape<2, 2>>();
+    case 16384: return wide_max_bins<WideShape<4, 4>>();
+    case 32768: return wide_max_bins<WideShape<8, 4>>();
+    case 65536: return wide_max_bins<WideShape<16, 8>>();
+    default: return 0;
+  }
+}
 
 long long wide_min_pairs(size_t n) { return kWideMinPairs[ilog2((int)n) - 13]; }
 

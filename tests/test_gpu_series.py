@@ -247,3 +247,30 @@ def test_series_forward_fills_data_rows(n, gpu_device):
     assert spec.shape == (nblk, n)
     with pytest.raises(RuntimeError):
         ctx.series_forward(series, starts, row0=2)        # rows 2..5 exceed ndata = 5
+
+
+@pytest.mark.parametrize("n,nblk,nt,bs", [(64, 5, 3, 64), (256, 64, 2, 40), (256, 65, 2, 40), (1024, 6, 9, 1024),
+                                          (4096, 5, 4, 4096), (4096, 4, 3, 512), (4096, 3, 2, 100), (8192, 3, 5, 8192),
+                                          (8192, 6, 50, 1000), (16384, 3, 90, 16384), (32768, 3, 2, 4096),
+                                          (32768, 5, 6, 4096), (65536, 4, 15, 65536), (1024, 3, 2, 1)])
+def test_a_window_per_block_matches_blocks_alone(n, nblk, nt, bs, gpu_device):
+    """Blocks with windows of their own (aligned, unaligned, touching the ends)
+    share one launch where the path allows it; every block must give what it
+    gives alone, bit for bit."""
+    rng = np.random.default_rng(n + nblk)
+    T = (rng.standard_normal((nt, n)) + 1j * rng.standard_normal((nt, n))).astype(np.complex64)
+    x = (rng.standard_normal(nblk * n // 2 + n) + 1j * rng.standard_normal(nblk * n // 2 + n)).astype(np.complex64)
+    starts = np.arange(nblk) * (n // 2)
+    for aligned in (True, False):
+        width = n // 2 if bs > 1 else 40
+        lo = np.array([(64 * (b % 5) if aligned else 7 * (b % 9)) % (n - width + 1) for b in range(nblk)])
+        hi = lo + width
+        if n >= 1024 and bs > 1:
+            hi[-1] = lo[-1] + width - (0 if aligned else 1) if bs < width else n
+        f = mf.MatchedFilter(n, 1, nt)
+        f.set_templates(T)
+        for thr in (0.0, 2.0 * float(np.sqrt(n)) / np.sqrt(n)):
+            got = f.run_series(x, starts, lo, hi, binsize=bs, threshold=thr)
+            for b in range(nblk):
+                one = f.run_series(x, starts[b:b + 1], lo[b:b + 1], hi[b:b + 1], binsize=bs, threshold=thr)
+                assert np.array_equal(got[b:b + 1], one), (n, b, aligned, thr)
