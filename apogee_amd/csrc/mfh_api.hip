@@ -66,6 +66,7 @@ Ctx::~Ctx() {
   if (stream) hipStreamDestroy(stream);
   if (stage) hipHostFree(stage);
   if (refine_hint) hipHostFree(refine_hint);
+  if (refined_host) hipHostFree(refined_host);
 }
 
 void *Ctx::host_stage(size_t bytes) {

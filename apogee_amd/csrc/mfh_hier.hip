@@ -97,31 +97,36 @@ __global__ void gate_kernel(const int64_t *cidx, const cf *cval, int nd, int nt,
 
 // Gate and refine in one launch after the FP32 screen (refine length FN, one
 // transform per 256-thread workgroup): each workgroup takes a tile of
-// kGateRows data rows x kGateTemplates templates, decides their gates in
+// kGatePairs pairs, `rows` data rows x kGatePairs / rows templates, decides their gates in
 // parallel by gate_kernel's rule from the screen's results, writes -1 / 0
 // into every bin of the dismissed pairs, clears the next call's counter,
 // runs the flat kernel's per-pair path on each survivor in turn, and adds
 // its survivors to this call's counter (one atomic per workgroup that has
 // any).  Replaces gate_kernel, the survivor list and the list-driven refine
 // launch.  A dense gate gives every workgroup at most 16 refines, whose rows
-// and templates are each read four times in a row.
-constexpr int kGateRows = 4, kGateTemplates = 4;
+// and templates are each read several times in a row.
+// The tile: a signal in one data row passes most of the bank, so a workgroup
+// refines as many pairs one after another as its tile has templates.  8 x 2
+// after a call with many survivors, else 4 x 4, whose results of dismissed
+// pairs leave in longer runs (public run, 16 x 1024, one row with a signal /
+// noise: 4 x 4 47.6 / 42.1 us, 8 x 2 42.3 / 45.0, 16 x 1 48.6 / 53.5).
+constexpr int kGatePairs = 16;
 template <int FN, int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, float thr, int *count, int *other,
+gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, int rows, float thr, int *count, int *other,
                    FlatArgs fa) {
   using S = FlatShape<FN>;
   static_assert(S::WG == 256 && S::SLOTS == 1 && S::TPT == 256, "one transform per 256-thread workgroup");
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int2 surv[kGateRows * kGateTemplates];
+  __shared__ int2 surv[kGatePairs];
   __shared__ int ns_sh;
   const int lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *other = 0;  // the next call's counter
   const int nb = (int)fa.nb;
   if (threadIdx.x < 64) {
-    const int d = blockIdx.y * kGateRows + lane / kGateTemplates;
-    const int tt = blockIdx.x * kGateTemplates + lane % kGateTemplates;
-    const bool inside = lane < kGateRows * kGateTemplates && d < nd && tt < nt;
+    const int d = blockIdx.y * rows + lane % rows;
+    const int tt = blockIdx.x * (kGatePairs / rows) + lane / rows;
+    const bool inside = lane < kGatePairs && d < nd && tt < nt;
     const long long p = (long long)d * nt + tt;
     bool fire = false;
     if (inside && cidx[p] >= 0) {
@@ -162,6 +167,15 @@ gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, float th
   // the count last: issued at the start, every workgroup's atomic on the one
   // counter would hold its refines back until it completed
   if (threadIdx.x == 0) atomicAdd(count, ns);
+}
+
+// A run's survivor count for the host: one small launch behind the run, in place
+// of a copy to pageable memory, for which the runtime stages, waits and copies
+// again (7 us of a public call).
+__global__ void refined_kernel(const int *count, long long *sum, long long *host, int first, int last) {
+  const long long s = (first ? 0 : *sum) + *count;
+  if (last) *host = s;
+  else *sum = s;
 }
 
 // Clears `n` ints (n <= 64), one workgroup: a kernel rather than a memset so
@@ -244,17 +258,33 @@ static int launch_gate_refine(Ctx *c, const int64_t *cidx, const cf *cval, int n
     return fail("the one-launch gate and refine does not apply here");
   using Kern = decltype(&gate_refine_kernel<FN, kOneBin>);
   const Kern kern = nb == 1 ? gate_refine_kernel<FN, kOneBin> : gate_refine_kernel<FN, kAligned>;
-  const dim3 grid((unsigned)((nt + kGateTemplates - 1) / kGateTemplates), (unsigned)((nd + kGateRows - 1) / kGateRows));
+  const int rows = c->many_refined((long long)nd * nt) ? 8 : 4;
+  const int templates = kGatePairs / rows;
+  const dim3 grid((unsigned)((nt + templates - 1) / templates), (unsigned)((nd + rows - 1) / rows));
   if (grid.y > 65535) return fail("too many data rows per launch (%d)", nd);
   const size_t smem = (size_t)FlatShape<FN>::XSTRIDE * sizeof(cf) + 2 * (size_t)nb * sizeof(uint64_t);
   if (!lds_limit((const void *)kern, c->dev, smem)) return -1;
   Ctx::ProfScope ps(c, "refine");
-  hipLaunchKernelGGL(kern, grid, dim3(256), smem, c->stream, cidx, cval, nd, nt, thr, count, other, fa);
+  hipLaunchKernelGGL(kern, grid, dim3(256), smem, c->stream, cidx, cval, nd, nt, rows, thr, count, other, fa);
   return hip_ok(hipGetLastError(), "gate_refine_kernel") ? 0 : -1;
 }
 
+static int deliver_refined(Ctx *c, const int *count, const RefinedOut &to) {
+  if (to.copy)
+    return hip_ok(hipMemcpyAsync(to.copy, count, sizeof(int), hipMemcpyDeviceToHost, c->stream), "copy count") ? 0 : -1;
+  if (!to.host) return 0;
+  long long *sum = (long long *)c->scratch("refined_sum", sizeof(long long));
+  if (!sum) return -1;
+  if (!c->refined_host &&
+      !hip_ok(hipHostMalloc((void **)&c->refined_host, sizeof(long long), hipHostMallocCoherent), "hipHostMalloc"))
+    return -1;
+  hipLaunchKernelGGL(refined_kernel, dim3(1), dim3(1), 0, c->stream, count, sum, c->refined_host, (int)to.first,
+                     (int)to.last);
+  return hip_ok(hipGetLastError(), "refined_kernel") ? 0 : -1;
+}
+
 int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-             float coarse_thr, const PeakOut &out, int *count_out, const cf *data_rows, const HierScratch *hs) {
+             float coarse_thr, const PeakOut &out, RefinedOut refined, const cf *data_rows, const HierScratch *hs) {
   if (c->coarse_band <= 0) return fail("no coarse band: call mfh_hier_set_band first");
   if (!(coarse_thr >= 0.f) || !std::isfinite(coarse_thr))
     return fail("coarse threshold must be finite and nonnegative");
@@ -319,10 +349,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
       if (launch_coarse_refine(c, drows, (long long)n, t0, nd, nt, (int)cs, (int)ce, c->coarse_prec == 2, g, rr) < 0)
         return -1;
       if (!c->capturing && !hs) c->hier_parity ^= 1;
-      if (count_out &&
-          !hip_ok(hipMemcpyAsync(count_out, count, sizeof(int), hipMemcpyDeviceToHost, c->stream), "copy count"))
-        return -1;
-      return 0;
+      return deliver_refined(c, count, refined);
     }
     if (launch_coarse_mfma(c, drows, (long long)n, t0, nd, nt, (int)cs, (int)ce, c->coarse_prec == 2, nullptr, &g) <
         0)
@@ -351,10 +378,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
       const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, out);
       if (launch_gate_refine(c, cidx, cval, nd, nt, coarse_thr, count, other, rr) < 0) return -1;
       if (!c->capturing && !hs) c->hier_parity ^= 1;
-      if (count_out &&
-          !hip_ok(hipMemcpyAsync(count_out, count, sizeof(int), hipMemcpyDeviceToHost, c->stream), "copy count"))
-        return -1;
-      return 0;
+      return deliver_refined(c, count, refined);
     }
     Ctx::ProfScope ps(c, "gate");
     hipLaunchKernelGGL(gate_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, c->stream, cidx, cval, nd,
@@ -379,10 +403,7 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
   }
   rr.hint = hs ? nullptr : c->refine_hint;
   if (launch_flat(c, n, rr) < 0) return -1;
-  if (count_out &&
-      !hip_ok(hipMemcpyAsync(count_out, count, sizeof(int), hipMemcpyDeviceToHost, c->stream), "copy count"))
-    return -1;
-  return 0;
+  return deliver_refined(c, count, refined);
 }
 
 }  // namespace mfh
@@ -507,9 +528,9 @@ static long long dbits(double x) {
 // launch parameters runs eagerly, the second identical call is captured into
 // a HIP graph, and later identical calls replay it with one launch.
 int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-                    float coarse_thr, const PeakOut &out, int *count_out) {
+                    float coarse_thr, const PeakOut &out, RefinedOut refined) {
   if (!c->use_graphs || c->prof_on)
-    return hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, count_out, nullptr);
+    return hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, refined, nullptr);
   hipSetDevice(c->dev);
   if (c->coarse_band > 0 && hier_prepare(c) < 0) return -1;
   std::vector<long long> key = {d0, nd, t0, nt, (long long)binsize, fbits(threshold), (long long)ws, (long long)we,
@@ -532,7 +553,7 @@ int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, floa
     if (!hip_ok(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
       return -1;
     c->capturing = true;
-    const int rc = hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, nullptr, nullptr);
+    const int rc = hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, RefinedOut{}, nullptr);
     c->capturing = false;
     const bool ended = hip_ok(hipStreamEndCapture(c->stream, &g), "hipStreamEndCapture");
     if (rc < 0 || !ended) {
@@ -547,17 +568,13 @@ int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, floa
     if (!hip_ok(hipGraphLaunch(ex, c->stream), "hipGraphLaunch")) return -1;
     c->hier_parity ^= 1;
   } else {
-    if (hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, nullptr, nullptr) < 0)
+    if (hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, RefinedOut{}, nullptr) < 0)
       return -1;
     c->last_key = key;
   }
-  if (count_out) {
-    int *count = hier_counter(c, par);
-    if (!count || !hip_ok(hipMemcpyAsync(count_out, count, sizeof(int), hipMemcpyDeviceToHost, c->stream),
-                          "copy count"))
-      return -1;
-  }
-  return 0;
+  if (!refined.copy && !refined.host) return 0;
+  int *count = hier_counter(c, par);
+  return count ? deliver_refined(c, count, refined) : -1;
 }
 
 }  // namespace mfh
@@ -568,7 +585,7 @@ extern "C" int mfh_hier_peaks_async(mfh_ctx *ctx, int d0, int nd, int t0, int nt
   if (!ctx) return fail("null context");
   Ctx *c = reinterpret_cast<Ctx *>(ctx);
   return mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr,
-                              mfh::peak_arrays(dev_idx, dev_val_c64), host_refined);
+                              mfh::peak_arrays(dev_idx, dev_val_c64), {host_refined});
 }
 
 static long hier_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws,
@@ -583,11 +600,10 @@ static long hier_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t
   if (nd < 1 || nt < 1) return fail("data/templates sub-range out of bounds");
   const size_t cells = (size_t)nd * (size_t)nt * nb;
   hipSetDevice(c->dev);
-  int refined = 0;
   mfh::PeakOut out;
   const bool direct = !c->use_graphs && mfh::host_results(cells, idx, val_c64, rec, out);
   if (!direct && !mfh::peak_buffer(c, cells, out)) return -1;
-  if (mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, &refined) < 0) {
+  if (mfh::hier_run_cached(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr, out, {nullptr, true}) < 0) {
     hipStreamSynchronize(c->stream);  // a launch before the failure may still write the caller's buffer
     return -1;
   }
@@ -595,7 +611,8 @@ static long hier_peaks_host(mfh_ctx *ctx, int d0, int nd, int t0, int nt, size_t
                             : mfh::read_peaks(c, out, cells, nb, idx, val_c64, counts, rec);
   if (total < 0) return -1;
   c->prof_collect();
-  if (n_refined) *n_refined = refined;
+  c->last_refined = mfh::refined_count(c);
+  if (n_refined) *n_refined = c->last_refined;
   return total;
 }
 
@@ -672,7 +689,7 @@ extern "C" int mfh_hier_peaks_noalloc(mfh_ctx *ctx, int d0, int nd, int t0, int 
   hs.list = (int2 *)(base + kNoAllocHead + pairs * (sizeof(int64_t) + sizeof(mfh::cf)));
   c->no_alloc = true;
   const int rc = mfh::hier_run(c, d0, nd, t0, nt, binsize, threshold, ws, we, coarse_thr,
-                               mfh::peak_arrays(dev_idx, dev_val_c64), nullptr, nullptr, &hs);
+                               mfh::peak_arrays(dev_idx, dev_val_c64), {}, nullptr, &hs);
   c->no_alloc = false;
   return rc;
 }

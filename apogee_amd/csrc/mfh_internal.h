@@ -68,6 +68,14 @@ struct Ctx {
   // pinned host word holding the last hierarchical refine's survivor count,
   // written by that launch (a sizing hint only: results never depend on it)
   int *refine_hint = nullptr;
+  // pinned host word that a hierarchical call's (or series') survivor count is
+  // left in for the host, and the device word that a series sums it in
+  long long *refined_host = nullptr;
+  // Whether the previous call with a count refined 1/64 of its pairs or more:
+  // the one-launch screens then cut their tiles for survivors that share a data
+  // row.  Any tile gives the same results.
+  long long last_refined = 0;
+  bool many_refined(long long pairs) const { return last_refined * 64 >= pairs; }
   // Per-pass twiddle tables of the flat kernel for length n (FP64-generated
   // on first use, kept for the context's lifetime).
   std::map<size_t, cf *> tw_by_n;
@@ -279,8 +287,18 @@ struct HierScratch {
   int *count = nullptr;
   int *spare = nullptr;
 };
+// Where a hierarchical run's survivor count goes: nowhere, to the caller's host
+// word by a copy on the stream, or to Ctx::refined_host by a kernel behind the
+// run, alone or as part of the sum over a series' groups.
+struct RefinedOut {
+  int *copy = nullptr;
+  bool host = false;                 // a kernel sums it for Ctx::refined_host
+  bool first = true, last = true;    // of the groups that are summed
+};
 int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
-             float coarse_thr, const PeakOut &out, int *count_out, const cf *data_rows,
+             float coarse_thr, const PeakOut &out, RefinedOut count, const cf *data_rows,
              const HierScratch *hs = nullptr);
+// The survivor count that RefinedOut::kHost left (after a stream wait).
+inline long long refined_count(const Ctx *c) { return *(volatile long long *)c->refined_host; }
 
 }  // namespace mfh

@@ -278,8 +278,6 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
     base.win_aligned = aligned;
   }
   if (mfh::launch_series_forward(c, dser, nseries, bs, nblocks, spec) < 0) return -1;
-  long long refined_total = 0;
-  std::vector<int> refined;
   // consecutive blocks with equal windows share one launch, and with `win`
   // all blocks do, each row reading its own
   for (int b0 = 0; b0 < nblocks;) {
@@ -288,14 +286,10 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
     const size_t ws = win_start[b0], we = std::min(win_end[b0], n);
     const mfh::PeakOut group = out.at((size_t)b0 * nt * nb);
     if (hier) {
-      refined.push_back(0);
-      // survivor counts are read from the device list counter per group
-      int cnt = 0;
-      if (mfh::hier_run(c, 0, g, t0, nt, binsize, threshold, ws, we, coarse_thr, group, &cnt,
-                        spec + (size_t)b0 * n) < 0 ||
-          !hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))
+      // the survivor counts are summed on the device over the groups
+      if (mfh::hier_run(c, 0, g, t0, nt, binsize, threshold, ws, we, coarse_thr, group,
+                        {nullptr, true, b0 == 0, b0 + g == nblocks}, spec + (size_t)b0 * n) < 0)
         return -1;
-      refined_total += cnt;
     } else {
       mfh::FlatRun r = base;
       r.data = spec + (size_t)b0 * n;
@@ -313,7 +307,8 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
   if (total < 0) return -1;
   wait_on_return.armed = false;
   c->prof_collect();
-  if (n_refined) *n_refined = refined_total;
+  if (hier) c->last_refined = mfh::refined_count(c);
+  if (n_refined) *n_refined = hier ? c->last_refined : 0;
   return total;
 }
 

@@ -439,3 +439,42 @@ def test_one_launch_screen_and_refine_matches_two_launches(prec, gpu_device):
                         assert ra == nd * nt, label
                     np.testing.assert_array_equal(a["index"], b["index"], err_msg=label)
                     np.testing.assert_array_equal(a["value"], b["value"], err_msg=label)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp16"])
+@pytest.mark.parametrize("nd", [1, 3, 16])
+def test_tiles_chosen_by_the_previous_call_give_the_same_results(prec, nd, gpu_device):
+    """A call with many survivors makes the next one cut its tiles differently:
+    signal, noise and signal again, against filters that run each once."""
+    n, nt = 4096, 130
+    rng = np.random.default_rng(nd)
+
+    def cnoise(rng, shape):
+        return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+
+    T = cnoise(rng, (nt, n))
+    T[:, 600:] *= 0.02
+    T /= np.linalg.norm(T, axis=1, keepdims=True)
+    T = T.astype(np.complex64)
+    noise = cnoise(rng, (nd, n))
+    loud = noise.copy()
+    loud[0] += (40.0 * T[::3].sum(axis=0)).astype(np.complex64)
+
+    def make():
+        h = mf.HierarchicalFilter(n, nd, nt, band=512)
+        h.set_coarse_threshold(5.0)
+        h.set_coarse_precision(prec)
+        h.set_templates(T)
+        return h
+
+    h = make()
+    for D in (loud, loud, noise, noise, loud):
+        once = make()
+        once.set_data(D)
+        h.set_data(D)
+        p0, r0 = h.stats
+        got = h.run(threshold=4.0)
+        assert np.array_equal(got, once.run(threshold=4.0))
+        assert h.stats[1] - r0 == once.stats[1]
+        if D is loud:
+            assert once.stats[1] * 64 >= nd * nt
