@@ -84,7 +84,6 @@ int launch_n(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, si
   FlatArgs a;
   if (flat_base_args(c, N, r, ws, we, nb_total, bin0, nb, a) < 0) return -1;
   const bool list = r.list != nullptr;
-  const int dpw = a.dpw;
   dim3 grid;
   if (list) {
     // enough workgroups to fill the device; each drains the list grid-stride.
@@ -99,8 +98,19 @@ int launch_n(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, si
     }
     grid = dim3((unsigned)std::max(1, std::min(want, c->refine_grid_cap)), 1);
   } else {
-    grid = dim3((unsigned)((r.nt + S::SLOTS - 1) / S::SLOTS), (unsigned)((r.nd + dpw - 1) / dpw));
-    if (grid.y > 65535) return fail("too many data rows per launch (%d)", r.nd);
+    if ((r.nd + a.dpw - 1) / a.dpw > 65535) return fail("too many data rows per launch (%d)", r.nd);
+    // A tile of several rows saves nothing but workgroups (the template is
+    // read again for each row, from the caches): one row per workgroup unless
+    // tuned otherwise (n = 4096, eight bins, calls with device results: 64 x 32
+    // pairs 46.7 us with tiles of four, which leave half of the chip idle,
+    // and 40.5 with one; 16 x 16 43.4 and 28.0; 64 x 512 256.6 and 246.5), and
+    // a tuned tile only while it leaves 1024 workgroups
+    const unsigned groups = (unsigned)((r.nt + S::SLOTS - 1) / S::SLOTS);
+    int dpw = c->tune_dpw > 0 ? c->tune_dpw : 1;
+    while (dpw > 1 && (long long)groups * ((r.nd + dpw - 1) / dpw) < 1024) dpw /= 2;
+    dpw = std::max(dpw, (r.nd + 65534) / 65535);
+    a.dpw = dpw;
+    grid = dim3(groups, (unsigned)((r.nd + dpw - 1) / dpw));
   }
   const size_t lds = flat_lds_bytes<N>(nb);
   int mode = kGeneral;
