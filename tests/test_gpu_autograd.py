@@ -173,3 +173,37 @@ def test_peak_fit_gradients(gpu_device):
             scale = np.abs(g_r[:, p]).max()
             assert abs(g[t, p] - fd) <= 1e-3 * abs(fd) + 1e-5 * scale, (t, p, g[t, p], fd)
             assert abs(g_r[t, p] - fd) <= 1e-5 * abs(fd) + 1e-7 * scale, (t, p, g_r[t, p], fd)
+
+
+@pytest.mark.parametrize("n,nd,nt,nb", [
+    (512, 3, 2, 3),         # below the matrix-core kernel
+    (1024, 1, 1, 1),        # one term, one tile per half
+    (1024, 2, 70, 5),       # templates split over workgroups for the data rows, ragged waves
+    (2048, 1, 65, 8),       # a last split with fewer rows
+    (4096, 3, 2, 65),       # more bins than a wave's lanes
+    (2048, 2, 1, 1030),     # more bins than a chunk
+    (65536, 2, 3, 2),       # the longest root tables
+])
+def test_gradient_kernels_match_the_fp64_oracle(gpu_device, n, nd, nt, nb):
+    # a term is about ten FP32 roundings (two roots, each a product of two;
+    # three products; its sums), 6e-7 relative at worst, and errors and terms
+    # grow alike with their number: 2e-6 of the largest element
+    from apogee_amd.autograd import PeakFilter
+    rng = np.random.default_rng(n + 7 * nd + nt + nb)
+    D, T, g = cnoise(rng, (nd, n)), cnoise(rng, (nt, n)), cnoise(rng, (nd, nt, nb))
+    idx = rng.integers(0, n, (nd, nt, nb))
+    idx[rng.random(idx.shape) < 0.2] = -1
+    idx[0, 0, 0] = n - 1
+    if nt > 1 and nd > 1:
+        idx[:, 1] = -1          # nothing reported: the row's NaN is not looked at
+        T[1, 5] = np.nan
+    g[idx < 0] = np.nan         # the gradient of an empty bin is not looked at
+    gpu = lambda x: torch.from_numpy(x).cuda()
+    pf = PeakFilter(n, nd, nt)
+    got = [pf._backward(gpu(D), gpu(T), gpu(idx), gpu(g), *need) for need in ((True, True), (True, False), (False, True))]
+    assert got[1][1] is None and got[2][0] is None
+    assert torch.equal(got[1][0], got[0][0]) and torch.equal(got[2][1], got[0][1])
+    gD, gT = O.peak_grads(D, np.nan_to_num(T), idx, np.nan_to_num(g))
+    for a, ref, what in ((got[0][0], gD, "data"), (got[0][1], gT, "templates")):
+        a = a.cpu().numpy().astype(np.complex128)
+        assert np.abs(a - ref).max() <= 2e-6 * np.abs(ref).max(), what
