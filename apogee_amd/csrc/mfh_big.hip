@@ -119,8 +119,17 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
 // The pair's rows and its Y block are wave-uniform, so loads and stores go
 // through buffer descriptors: one vector offset per thread and the per-u
 // stride as a scalar offset, with no vector address arithmetic per point.
+// A workgroup keeps its columns and walks pairs, so the closing twiddles are
+// found once and the next pair's template columns, which come from HBM, are
+// read into registers while this pair is transformed and stored.  One tile
+// per workgroup, all in step, first read, then wrote: n = 262144, 2 x 31 pairs,
+// cold templates: 63.2 us, of which reading alone takes 35 and writing alone
+// 23; with the walk 53.0 (195 MB, 3.7 TB/s; the same at three or four
+// workgroups per CU and with the data columns read ahead too).  At 4 waves per SIMD
+// the registers spill (59.9 us).
 template <class B>
-__global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu(4))) big_cols_kernel(BigArgs a) {
+__global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu(3)))
+big_cols_kernel(BigArgs a, int np) {
   constexpr int N = B::N, ROW = B::ROW, CT = B::CT;
   extern __shared__ __align__(16) unsigned char smem[];
   const int s = threadIdx.x & 15;
@@ -132,40 +141,72 @@ __global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu
   // as bt[17 s + u] (rows of 17: the 16 columns a wave reads in one step
   // fall in distinct banks, its 4 row groups read the same words).
   cf *bt = reinterpret_cast<cf *>(smem) + 16 * B::COL_STRIDE;
-  const long long pl = blockIdx.y;  // pair within the chunk
   if (a.hint && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.hint = *a.list_count;
-  int d = 0, tt = 0;
-  const bool valid = big_pair(a, a.p0 + pl, d, tt);  // uniform across the workgroup
-  if (!valid) return;                                 // no barrier has run yet
+  const int count = (int)min((long long)np, (a.list ? (long long)*a.list_count : (long long)a.nd * a.nt) - a.p0);
+  int pl = (int)blockIdx.y;  // pair within the chunk
+  if (pl >= count) return;  // uniform; no barrier has run yet
   const int f1 = blockIdx.x * 16 + s;
   cf wt{1.f, 0.f};
   if constexpr (!B::RF) {
     bt[17 * s + t] = big_root(a, 16 * f1 * t);  // u = t; 16 f1 t < n
     wt = big_root(a, f1 * t);
   }
-  const cf *D = uniform_ptr(a.data + (long long)d * a.data_stride);
-  const cf *T = uniform_ptr(a.tmpl + (long long)tt * a.tmpl_stride);
-  const __amdgpu_buffer_rsrc_t rd =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<cf *>(D), (short)0, N * (int)sizeof(cf), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rt =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<cf *>(T), (short)0, N * (int)sizeof(cf), 0x00020000);
-  const int voff = (f1 + ROW * t) * (int)sizeof(cf);  // element f1 + ROW (t + CT u) at voff + u * CT ROW * 8
-  cf v[16];
-#pragma unroll
-  for (int u = 0; u < 16; u++) {
-    const int so = u * CT * ROW * (int)sizeof(cf);
-    const cf x = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rd, voff, so, 0));
-    const cf y = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rt, voff, so, 0));
-    v[u] = cmul_conj(x, y);
+  cf w1{1.f, 0.f}, w4{1.f, 0.f};  // the column passes' twiddles depend on t only
+  if constexpr (B::ROWS == 256) {
+    w1 = a.twCol[TwiddleLayout<256>::offset(1) + t];
+    w4 = a.twCol[TwiddleLayout<256>::offset(1) + 16 + t];
   }
-  inverse_fft<B::ROWS>(v, t, xch, a.twCol);  // its barriers order the bt stores before the reads
-  cf *Y = const_cast<cf *>(uniform_ptr(a.scratch + pl * N));
-  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(Y, (short)0, N * (int)sizeof(cf), 0x00020000);
-  const int yoff = (t * ROW + f1) * (int)sizeof(cf);  // Y[k2][f1], k2 = t + CT u
+  const int voff = (f1 + ROW * t) * (int)sizeof(cf);  // element f1 + ROW (t + CT u) at voff + u * CT ROW * 8
+  auto row_rsrc = [](const cf *row) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<cf *>(uniform_ptr(row)), (short)0, N * (int)sizeof(cf),
+                                             0x00020000);
+  };
+  auto load = [&](cf *x, __amdgpu_buffer_rsrc_t r) {
 #pragma unroll
-  for (int u = 0; u < 16; u++) {
-    if constexpr (!B::RF) v[u] = cmul(v[u], cmul(wt, bt[17 * s + u]));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[u]), ry, yoff, u * CT * ROW * (int)sizeof(cf), 0);
+    for (int u = 0; u < 16; u++)
+      x[u] = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(r, voff, u * CT * ROW * (int)sizeof(cf), 0));
+  };
+  int d = 0, tt = 0;
+  big_pair(a, a.p0 + pl, d, tt);
+  cf y[16];
+  load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
+  for (;;) {
+    cf v[16];
+    load(v, row_rsrc(a.data + (long long)d * a.data_stride));
+    const int next = pl + (int)gridDim.y;
+    const bool more = next < count;
+    if (more) big_pair(a, a.p0 + next, d, tt);
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = cmul_conj(v[u], y[u]);
+    // the next pair's template is read while this one is transformed and stored
+    if (more) load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
+    __builtin_amdgcn_sched_barrier(0);
+    // the transform's barriers order the bt stores before the reads
+    if constexpr (B::ROWS == 256) {
+      dft16(v);
+      stockham_store<256, 16, 1>(v, t, xch);
+      __syncthreads();
+      stockham_load<256>(v, t, xch);
+      cf w[15];
+      power_twiddles(w, w1, w4);
+#pragma unroll
+      for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
+      dft16(v);
+    } else {
+      inverse_fft<B::ROWS>(v, t, xch, a.twCol);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const __amdgpu_buffer_rsrc_t ry = row_rsrc(a.scratch + (long long)pl * N);
+    const int yoff = (t * ROW + f1) * (int)sizeof(cf);  // Y[k2][f1], k2 = t + CT u
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      if constexpr (!B::RF) v[u] = cmul(v[u], cmul(wt, bt[17 * s + u]));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[u]), ry, yoff, u * CT * ROW * (int)sizeof(cf),
+                                            0);
+    }
+    if (!more) break;
+    pl = next;
+    __syncthreads();  // the exchange is read
   }
 }
 
@@ -344,6 +385,7 @@ __global__ void roots_kernel(cf *out, int L, int period) {
 }
 
 constexpr size_t kLds = 160 * 1024;
+constexpr int kColGrid = 1024;  // columns workgroups per launch: four per CU, of which three are resident at a time
 
 template <class B>
 size_t rows_max_bins() {
@@ -430,7 +472,9 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
       a.pkey = pkey2 + (ci & 1) * part_cells;
       a.pval = pval2 + (ci & 1) * part_cells;
     }
-    hipLaunchKernelGGL(big_cols_kernel<B>, dim3(B::ROW / 16, (unsigned)np), dim3(16 * B::CT), lds_cols, c->stream, a);
+    const unsigned walkers = (unsigned)std::min<long long>(np, kColGrid / (B::ROW / 16));
+    hipLaunchKernelGGL(big_cols_kernel<B>, dim3(B::ROW / 16, walkers), dim3(16 * B::CT), lds_cols, c->stream, a,
+                       (int)np);
     if (!hip_ok(hipGetLastError(), "big_cols_kernel")) return -1;
     a.hint = nullptr;
     for (size_t b0 = 0; b0 < nb_total; b0 += maxb) {

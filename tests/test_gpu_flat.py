@@ -559,6 +559,23 @@ def test_lengths_beyond_the_reference_gpu_set(n, gpu_device):
                            context="n=%d binsize=%d" % (n, binsize))
 
 
+@pytest.mark.parametrize("n,nd,nt", [(131072, 3, 13), (1048576, 1, 6)])
+def test_more_pairs_than_column_workgroups(n, nd, nt, gpu_device):
+    """Workgroups that walk several pairs, the last walk shorter, leave what a
+    call of one pair does."""
+    rng = np.random.default_rng(n + nt)
+    D, T = cnoise(rng, (nd, n)), cnoise(rng, (nt, n))
+    f = mf.MatchedFilter(n, nd, nt, device="gpu")
+    f.set_data(D)
+    f.set_templates(T)
+    whole = f.run(binsize=n // 8, threshold=0.0)
+    assert_peaks_match(D, T, whole["index"], whole["value"], n // 8, 0.0, None, context="n=%d" % n)
+    for d in range(nd):
+        for t in range(nt):
+            one = f.run(binsize=n // 8, threshold=0.0, data=(d, 1), templates=(t, 1))
+            assert np.array_equal(one[0, 0], whole[d, t]), (d, t)
+
+
 def test_records_own_their_page_locked_buffers(gpu_device, monkeypatch):
     """run() records come from pooled page-locked buffers the device writes
     directly (mfh_host_alloc): a result held across calls keeps its values,

@@ -97,6 +97,14 @@ def test_every_transform_length(n, gpu_device):
     assert_one_sided(a, b, "n=%d" % n)
 
 
+def test_survivors_beyond_the_column_workgroups(gpu_device):
+    # every pair has samples beyond 3, and the screen lets a good part of the 400
+    # through, against 32 workgroups per column block
+    a, b, _ = run_both(131072, 4, 100, 131072 // 8, 3.0, None)
+    fired = assert_one_sided(a, b, "400 pairs")
+    assert fired.any(axis=-1).sum() > 32
+
+
 @pytest.mark.parametrize("threshold", [3.0, 5.5, 8.0, 20.0])
 def test_thresholds(threshold, gpu_device):
     a, b, _ = run_both(4096, 2, 4, 512, threshold, None)
