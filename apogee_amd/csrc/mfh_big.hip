@@ -219,7 +219,8 @@ __device__ __forceinline__ void closing_passes(cf *v, int t, int k, cf *xch, con
   constexpr int p0 = L::NS0 == 1 ? 1 : 0;  // the table of NS = RF
   const cf *tw3 = tw + L::offset(p0 + 1), *tw4 = tw + L::offset(p0 + 2);
   cf w[15];
-  power_twiddles(w, tw3[k], tw3[16 * RF + k]);
+  const cf *e = tw + L::extra() + k;
+  power_twiddles(w, tw3[k], e[0], tw3[16 * RF + k], e[16 * RF]);
 #pragma unroll
   for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
   dft16(v);

@@ -143,12 +143,12 @@ int launch_len(Ctx *c, const FlatRun &r) {
   return 0;
 }
 
-// Rows r = 1, 4 of exp(+2 pi i r k / (16 ns)), k < ns, at [row][k],
+// Rows r = r0, 4 r0 of exp(+2 pi i r k / (16 ns)), k < ns, at [row][k],
 // generated in FP64.
-__global__ void twiddle_pass_kernel(cf *out, int ns) {
+__global__ void twiddle_pass_kernel(cf *out, int ns, int r0) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < ns * kTwiddleRows) {
-    const int r = i < ns ? 1 : 4, k = i % ns;
+    const int r = i < ns ? r0 : 4 * r0, k = i % ns;
     double s, c;
     sincospi(2.0 * (double)r * (double)k / (double)(16 * ns), &s, &c);
     out[i] = cf{(float)c, (float)s};
@@ -164,7 +164,12 @@ int fill_twiddles(Ctx *c, cf *tw) {
     if (ns == 1) continue;
     const int cnt = ns * kTwiddleRows;
     hipLaunchKernelGGL(twiddle_pass_kernel, dim3((cnt + 255) / 256), dim3(256), 0, c->stream,
-                       tw + L::offset(p), ns);
+                       tw + L::offset(p), ns, 1);
+  }
+  if (L::EXTRA_NS) {
+    const int cnt = L::EXTRA_NS * kTwiddleRows;
+    hipLaunchKernelGGL(twiddle_pass_kernel, dim3((cnt + 255) / 256), dim3(256), 0, c->stream, tw + L::extra(),
+                       L::EXTRA_NS, 2);
   }
   return hip_ok(hipGetLastError(), "twiddle launch") ? 0 : -1;
 }

@@ -252,29 +252,33 @@ __device__ __forceinline__ void wide_exchange(cf *v, int t, float *x) {
 }
 
 // Twiddles of butterflies Q0 .. Q0 + NQ - 1: register q + 2 r times w^r, with
-// the powers from the table rows w^1 and w^4 by load_twiddles16's products,
+// the powers from the table rows w^1, w^4 (and w^2, w^8) by power_twiddles' products,
 // each used as soon as it is known (w^1 ... w^8 are all that stays live).
 template <int Q0, int NQ>
-__device__ __forceinline__ void wide_twiddle(cf *v, cf w1, cf w4) {
+__device__ __forceinline__ void wide_twiddle(cf *v, cf w1, cf w2, cf w4, cf w8) {
   auto use = [&](int r, cf w) {
 #pragma unroll
     for (int q = Q0; q < Q0 + NQ; q++) v[q + 2 * r] = cmul(v[q + 2 * r], w);
   };
   cf w[8];
   w[1] = w1;
-  w[2] = cmul(w1, w1);
+  w[2] = w2;
   w[3] = cmul(w1, w[2]);
   w[4] = w4;
   w[5] = cmul(w1, w4);
   w[6] = cmul(w[2], w4);
   w[7] = cmul(w[3], w4);
-  const cf w8 = cmul(w4, w4);
   use(8, w8);
 #pragma unroll
   for (int r = 1; r < 8; r++) {
     use(r, w[r]);
     use(r + 8, cmul(w[r], w8));
   }
+}
+
+template <int Q0, int NQ>
+__device__ __forceinline__ void wide_twiddle(cf *v, cf w1, cf w4) {
+  wide_twiddle<Q0, NQ>(v, w1, cmul(w1, w1), w4, cmul(w4, w4));
 }
 
 // One radix-16 butterfly in place, registers q + 2 r.
@@ -310,8 +314,14 @@ __device__ __forceinline__ void wide_transform(cf *v, int t, int h, float *x, co
   wide_exchange<W, 2>(v, t, x);
   wide_fence();
   {
-    const cf *p = tw3 + S * (t % (16 * FL)) + h;
-    wide_twiddle<0, 2>(v, p[0], p[16 * RF]);
+    const int k = S * (t % (16 * FL)) + h;
+    const cf *p = tw3 + k;
+    if constexpr (L::EXTRA_NS > 0) {
+      const cf *e = tw + L::extra() + k;
+      wide_twiddle<0, 2>(v, p[0], e[0], p[16 * RF], e[16 * RF]);
+    } else {
+      wide_twiddle<0, 2>(v, p[0], p[16 * RF]);
+    }
   }
   wide_fence();
   wide_dft16(v, 0);
