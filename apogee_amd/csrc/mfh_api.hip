@@ -277,6 +277,15 @@ void *Ctx::scratch(const char *name, size_t bytes) {
   return b.p;
 }
 
+int *Ctx::part_counters(size_t pairs) {
+  const size_t bytes = pairs * sizeof(int);
+  const auto found = bufs.find("part_done");
+  const bool ready = found != bufs.end() && found->second.p && found->second.bytes >= bytes;
+  int *p = (int *)scratch("part_done", bytes);
+  if (p && !ready && !hip_ok(hipMemsetAsync(p, 0, bytes, stream), "hipMemsetAsync")) return nullptr;
+  return p;
+}
+
 int Ctx::own_bank(bool templates) {
   cf *&cur = templates ? tmpl : data;
   cf *own = templates ? tmpl_own : data_own;

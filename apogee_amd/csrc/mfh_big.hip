@@ -62,6 +62,7 @@ struct BigArgs {
   int nsplit;               // rows workgroups per pair (gridDim.y of the rows kernel)
   uint64_t *pkey;           // nsplit > 1: per-part bin tables [pair][part][nb]
   cf *pval;
+  int *done;                // if set: the pair's last part merges them (part_is_last); else finish_cell's launches
   PeakOut out;
   uint32_t ws, we, binsize, nb, ostride;
   int bshift;
@@ -89,10 +90,34 @@ __device__ __forceinline__ cf big_root(const BigArgs &a, int m) { return cmul(a.
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// One (pair, bin) cell of a chunk whose rows launch left per-part tables:
-// the largest key over the parts (keys are distinct per lag, so exactly one
-// part holds it) and that part's value.  The keys are read first, all
-// independent loads, then the one value.
+// One bin of a pair (of the chunk) whose parts have left their tables: the
+// largest key over the parts (keys are distinct per lag, so exactly one
+// part holds it) and that part's value, to output element o.  The keys are
+// read first, all independent loads, then the one value.
+__device__ __forceinline__ void merge_cell(const BigArgs &a, long long pl, int b, long long o) {
+  const int nb = (int)a.nb;
+  const uint64_t *keys = a.pkey + pl * a.nsplit * (long long)nb + b;
+  uint64_t best = 0ull;
+  int bw = 0;
+#pragma unroll 8
+  for (int w = 0; w < a.nsplit; w++) {
+    const uint64_t key = part_get(keys + (long long)w * nb);
+    bw = key > best ? w : bw;
+    best = key > best ? key : best;
+  }
+  if (best)
+    a.out.put(o, (long long)(~(uint32_t)best),
+              __builtin_bit_cast(cf, part_get((const uint64_t *)a.pval + (pl * a.nsplit + bw) * (long long)nb + b)));
+  else
+    a.out.none(o);
+}
+
+// Where a pair's outputs start.
+__device__ __forceinline__ long long pair_out(const BigArgs &a, long long pl, int d, int t) {
+  return a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + t) * a.ostride;
+}
+
+// One (pair, bin) cell of a chunk after its rows launch.
 __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long long i) {
   const int nb = (int)a.nb;
   if (i >= np * nb) return;
@@ -100,18 +125,7 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
   const int b = (int)(i % nb);
   int d = 0, tt = 0;
   if (!big_pair(a, a.p0 + pl, d, tt)) return;
-  const uint64_t *keys = a.pkey + pl * a.nsplit * (long long)nb + b;
-  uint64_t best = 0ull;
-  int bw = 0;
-#pragma unroll 8
-  for (int w = 0; w < a.nsplit; w++) {
-    const uint64_t key = keys[(long long)w * nb];
-    bw = key > best ? w : bw;
-    best = key > best ? key : best;
-  }
-  const long long o = a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-  if (best) a.out.put(o + b, (long long)(~(uint32_t)best), a.pval[(pl * a.nsplit + bw) * (long long)nb + b]);
-  else a.out.none(o + b);
+  merge_cell(a, pl, b, pair_out(a, pl, d, tt) + b);
 }
 
 // Columns: 16 columns f1 of one pair per workgroup; lane = 16 * t + s, so the
@@ -238,8 +252,9 @@ __device__ __forceinline__ void closing_passes(cf *v, int t, int k, cf *xch, con
 // Rows: nsplit workgroups per pair (workgroup = pair * nsplit + part), each
 // walking its share of the rows k2, SLOTS rows at a time.  With one part
 // the table is the result; with several, each part leaves its (key, value)
-// table, and finish_cell keeps the largest key per bin: in the next chunk's
-// rows launch, or in big_rows_finish_kernel after the last chunk.
+// table and merge_cell keeps the largest key per bin: in the pair's last part
+// or, for large tables, by finish_cell in the next chunk's rows launch or in
+// big_rows_finish_kernel after the last chunk.
 template <class B>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
@@ -352,16 +367,18 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
     }
     __syncthreads();  // values settled before the next group raises keys; xch reusable
   }
+  const long long o = pair_out(a, pl, d, tt);
   if (a.nsplit > 1) {
     const long long po = (pl * a.nsplit + part) * (long long)nb;
     for (int b = threadIdx.x; b < nb; b += 256) {
       const uint64_t key = bkey[b];
-      a.pkey[po + b] = key;
-      a.pval[po + b] = key ? bval[b] : cf{0.f, 0.f};
+      part_put(a.pkey + po + b, key);
+      part_put((uint64_t *)a.pval + po + b, key ? __builtin_bit_cast(uint64_t, bval[b]) : 0ull);
     }
+    if (a.done && part_is_last(a.done + pl, a.nsplit, *reinterpret_cast<int *>(smem)))
+      for (int b = threadIdx.x; b < nb; b += 256) merge_cell(a, pl, b, o + b);
     return;
   }
-  const long long o = a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
   for (int b = threadIdx.x; b < nb; b += 256) {
     const uint64_t key = bkey[b];
     if (key) a.out.put(o + b, (long long)(~(uint32_t)key), bval[b]);
@@ -386,6 +403,10 @@ __global__ void roots_kernel(cf *out, int L, int period) {
 }
 
 constexpr size_t kLds = 160 * 1024;
+// Table entries that a pair's last part merges: n = 262144, 2 x 31 pairs, 64 bins x
+// 16 parts 104.0 us a call against 105.8 with finish_cell, 512 x 16 110.7
+// against 116.2; 131072, 2 x 10, 2048 x 32: 67.5 against 56.8.  One pair: 35.4 and 36.4.
+constexpr size_t kMergeCells = 8192;
 constexpr int kColGrid = 1024;  // columns workgroups per launch: four per CU, of which three are resident at a time
 
 template <class B>
@@ -458,8 +479,15 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
     pval2 = (cf *)c->scratch("big_part_val", 2 * part_cells * sizeof(cf));
     if (!pkey2 || !pval2) return -1;
   }
-  // the finish of a chunk runs in the next rows launch when the window is
-  // one piece (one rows launch per chunk); else after each rows launch
+  // a pair's last part merges the tables where that is little work for one
+  // workgroup; else the finish of a chunk runs in the next rows launch when the
+  // window is one piece (one rows launch per chunk), and after each rows launch when not
+  a.done = nullptr;
+  if (nsplit > 1) {
+    a.done = c->part_counters((size_t)chunk);  // in any case: a later, captured call may have fewer bins
+    if (!a.done) return -1;
+    if (nb_piece * nsplit > kMergeCells) a.done = nullptr;
+  }
   const bool fold = nsplit > 1 && nb_total <= maxb;
   BigArgs fin = a;
   long long fin_np = 0;
@@ -491,7 +519,7 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
                          fin, fin_np, fin_blocks);
       if (!hip_ok(hipGetLastError(), "big_rows_kernel")) return -1;
       fin_blocks = 0;
-      if (nsplit > 1) {
+      if (nsplit > 1 && !a.done) {
         const long long cells = np * (long long)cnt;
         if (fold) {  // finished by the next rows launch, or after the loop
           fin = a;

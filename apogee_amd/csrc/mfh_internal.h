@@ -94,6 +94,8 @@ struct Ctx {
   std::map<std::string, Buf> bufs;
   // Device buffer `name`, grown on demand (contents not preserved on growth).
   void *scratch(const char *name, size_t bytes);
+  // one counter per pair of a launch for part_is_last, 0 between launches
+  int *part_counters(size_t pairs);
 
   // per-kernel event timing
   struct Ev {

@@ -58,6 +58,7 @@ struct WideArgs {
   long long np;            // pairs of this launch, at most
   uint64_t *pkey;          // S > 1: per-part bin tables [pair of the launch][part][nb]
   cf *pval;
+  int *done;               // tiled, S > 1: part_is_last's counter per pair of the launch
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -478,7 +479,7 @@ __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples 
   constexpr int S = W::S, T = W::T;
   auto put = [&](int b, uint32_t k, cf z) {
     if constexpr (S == 1) a.out.put(o + b, (long long)k, z);
-    else pval[o + b] = z;
+    else part_put((uint64_t *)pval + o + b, __builtin_bit_cast(uint64_t, z));
   };
   if (ONE || nb <= kWideLook) {
     const int w0 = __builtin_amdgcn_readfirstlane(t);
@@ -507,6 +508,26 @@ __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples 
       }
     }
   }
+}
+
+// One (pair, bin) cell: the largest key over the parts (keys are distinct per
+// lag) and that part's value.
+template <int S>
+__device__ __forceinline__ void wide_cell(const WideArgs &wa, long long pl, int b, long long o) {
+  const int nb = (int)wa.f.nb;
+  uint64_t best = 0ull;
+  int bw = 0;
+#pragma unroll
+  for (int h = 0; h < S; h++) {
+    const uint64_t key = part_get(wa.pkey + (pl * S + h) * nb + b);
+    bw = key > best ? h : bw;
+    best = key > best ? key : best;
+  }
+  if (best)
+    wa.f.out.put(o, (long long)(~(uint32_t)best),
+                 __builtin_bit_cast(cf, part_get((const uint64_t *)wa.pval + (pl * S + bw) * nb + b)));
+  else
+    wa.f.out.none(o);
 }
 
 template <class W, bool ONE, bool DENSE, bool LIST>
@@ -583,46 +604,33 @@ __global__ void __launch_bounds__(W::T) __attribute__((amdgpu_waves_per_eu(4))) 
     else o = (LIST && a.list_ooff) ? a.list_ooff[wa.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
     if (hot) wide_write<W, ONE>(a, WideSamples(v), hot, t, h, lane, nb, bins, o, wa.pval);
     for (int b = threadIdx.x; b < nb; b += T) {
-      if constexpr (S > 1) wa.pkey[o + b] = bins[b];
+      if constexpr (S > 1) part_put(wa.pkey + o + b, bins[b]);
       else if (bins[b] == 0ull) a.out.none(o + b);
+    }
+    if constexpr (S > 1 && !LIST) {
+      if (part_is_last(wa.done + pl, S, *reinterpret_cast<int *>(smem))) {
+        const long long ro = ((long long)d * a.nt + tt) * a.ostride;
+        for (int b = threadIdx.x; b < nb; b += T) wide_cell<S>(wa, pl, b, ro + b);
+      }
     }
     if constexpr (LIST) __syncthreads();  // the space is free for the next unit's exchange
     w += gridDim.x;
   } while (LIST && w < units);
 }
 
-// One (pair, bin) cell: the largest key over the parts (keys are distinct per
-// lag) and that part's value.
-template <int S, bool LIST>
+// The cells of a list launch.  Its workgroups go on to further pairs, one at a time
+// per CU, and would wait for their tables to arrive each time: 65536-point
+// requests of a mixed queue take 340 us with this launch and 347 without.
+template <int S>
 __global__ void __launch_bounds__(256) wide_finish_kernel(WideArgs wa) {
   const FlatArgs &a = wa.f;
-  const int nb = (int)a.nb;
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long pl = i / nb;
-  const int b = (int)(i % nb);
-  long long pairs = wa.np;
-  if constexpr (LIST) pairs = min(pairs, (long long)*a.list_count - wa.p0);
-  if (pl >= pairs) return;
-  int d, tt;
-  if constexpr (LIST) {
-    const int2 pr = a.list[wa.p0 + pl];
-    d = pr.x;
-    tt = pr.y;
-  } else {
-    tt = (int)((wa.p0 + pl) / a.nd);
-    d = (int)((wa.p0 + pl) % a.nd);
-  }
-  uint64_t best = 0ull;
-  int bw = 0;
-#pragma unroll
-  for (int h = 0; h < S; h++) {
-    const uint64_t key = wa.pkey[(pl * S + h) * nb + b];
-    bw = key > best ? h : bw;
-    best = key > best ? key : best;
-  }
-  const long long o = (LIST && a.list_ooff) ? a.list_ooff[wa.p0 + pl] : ((long long)d * a.nt + tt) * a.ostride;
-  if (best) a.out.put(o + b, (long long)(~(uint32_t)best), wa.pval[(pl * S + bw) * nb + b]);
-  else a.out.none(o + b);
+  const long long pl = i / (int)a.nb;
+  const int b = (int)(i % (int)a.nb);
+  if (pl >= min(wa.np, (long long)*a.list_count - wa.p0)) return;
+  const int2 pr = a.list[wa.p0 + pl];
+  const long long o = a.list_ooff ? a.list_ooff[wa.p0 + pl] : ((long long)pr.x * a.nt + pr.y) * a.ostride;
+  wide_cell<S>(wa, pl, b, o + b);
 }
 
 template <class W>
@@ -648,7 +656,8 @@ int wide_tables(Ctx *c, WideArgs &wa, long long total, size_t nb, long long &chu
   const size_t cells = (size_t)chunk * W::S * nb;
   wa.pkey = (uint64_t *)c->scratch("wide_key", cells * sizeof(uint64_t));
   wa.pval = (cf *)c->scratch("wide_val", cells * sizeof(cf));
-  return wa.pkey && wa.pval ? 0 : -1;
+  wa.done = c->part_counters((size_t)chunk);
+  return wa.pkey && wa.pval && wa.done ? 0 : -1;
 }
 
 template <class W, bool LIST>
@@ -668,10 +677,9 @@ int wide_piece(Ctx *c, WideArgs &wa, long long total, size_t nb) {
     if (!hip_ok(hipGetLastError(), "wide_kernel")) return -1;
     wa.f.zero = nullptr;
     wa.f.hint = nullptr;
-    if (W::S > 1) {
+    if (W::S > 1 && LIST) {
       const long long cells = wa.np * (long long)nb;
-      hipLaunchKernelGGL((wide_finish_kernel<W::S, LIST>), dim3((unsigned)((cells + 255) / 256)), dim3(256), 0,
-                         c->stream, wa);
+      hipLaunchKernelGGL(wide_finish_kernel<W::S>, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, c->stream, wa);
       if (!hip_ok(hipGetLastError(), "wide_finish_kernel")) return -1;
     }
   }

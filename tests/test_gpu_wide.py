@@ -97,3 +97,20 @@ def test_refine_lists_agree(n, gpu_device):
             h._gpu.set_tuning("wide", 0)
             for _ in range(2):
                 assert np.array_equal(a, h.run(binsize=bs, threshold=thr))
+
+
+@pytest.mark.parametrize("n,nd,nt", [(32768, 3, 11), (65536, 3, 5), (262144, 1, 5)])
+def test_parts_merge_alike_every_time(n, nd, nt, gpu_device):
+    """Pairs whose parts run on different XCDs, merged by whichever part comes
+    last: repeated calls, and calls of another shape between them, agree."""
+    D, T = bank(n, nd, nt, n + 3)
+    f = mf.MatchedFilter(n, nd, nt)
+    f.set_data(D)
+    f.set_templates(T)
+    if n <= 65536:
+        f._gpu.set_tuning("wide", ALWAYS)
+    first = f.run(binsize=n // 16)
+    assert_peaks_match(D, T, first["index"], first["value"], n // 16, 0.0, None, context=str(n))
+    for i in range(40):
+        assert np.array_equal(f.run(binsize=n // 16), first), i
+        f.run(binsize=n // 8, data=(0, 1), templates=(i % nt, 1))
