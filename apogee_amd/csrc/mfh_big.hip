@@ -62,7 +62,7 @@ struct BigArgs {
   int nsplit;               // rows workgroups per pair (gridDim.y of the rows kernel)
   uint64_t *pkey;           // nsplit > 1: per-part bin tables [pair][part][nb]
   cf *pval;
-  int *done;                // if set: the pair's last part merges them (part_is_last); else finish_cell's launches
+  int *done;                // RF > 0, if set: the pair's last part merges them (part_is_last)
   PeakOut out;
   uint32_t ws, we, binsize, nb, ostride;
   int bshift;
@@ -90,34 +90,14 @@ __device__ __forceinline__ cf big_root(const BigArgs &a, int m) { return cmul(a.
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// One bin of a pair (of the chunk) whose parts have left their tables: the
-// largest key over the parts (keys are distinct per lag, so exactly one
-// part holds it) and that part's value, to output element o.  The keys are
-// read first, all independent loads, then the one value.
-__device__ __forceinline__ void merge_cell(const BigArgs &a, long long pl, int b, long long o) {
-  const int nb = (int)a.nb;
-  const uint64_t *keys = a.pkey + pl * a.nsplit * (long long)nb + b;
-  uint64_t best = 0ull;
-  int bw = 0;
-#pragma unroll 8
-  for (int w = 0; w < a.nsplit; w++) {
-    const uint64_t key = part_get(keys + (long long)w * nb);
-    bw = key > best ? w : bw;
-    best = key > best ? key : best;
-  }
-  if (best)
-    a.out.put(o, (long long)(~(uint32_t)best),
-              __builtin_bit_cast(cf, part_get((const uint64_t *)a.pval + (pl * a.nsplit + bw) * (long long)nb + b)));
-  else
-    a.out.none(o);
-}
-
 // Where a pair's outputs start.
 __device__ __forceinline__ long long pair_out(const BigArgs &a, long long pl, int d, int t) {
   return a.list_ooff ? a.list_ooff[a.p0 + pl] : ((long long)d * a.nt + t) * a.ostride;
 }
 
-// One (pair, bin) cell of a chunk after its rows launch.
+// One (pair, bin) cell of a chunk after its rows launch: the largest key over
+// the parts (keys are distinct per lag, so exactly one part holds it) and that
+// part's value.  The keys are read first, all independent loads, then the one value.
 __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long long i) {
   const int nb = (int)a.nb;
   if (i >= np * nb) return;
@@ -125,7 +105,18 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
   const int b = (int)(i % nb);
   int d = 0, tt = 0;
   if (!big_pair(a, a.p0 + pl, d, tt)) return;
-  merge_cell(a, pl, b, pair_out(a, pl, d, tt) + b);
+  const uint64_t *keys = a.pkey + pl * a.nsplit * (long long)nb + b;
+  uint64_t best = 0ull;
+  int bw = 0;
+#pragma unroll 8
+  for (int w = 0; w < a.nsplit; w++) {
+    const uint64_t key = keys[(long long)w * nb];
+    bw = key > best ? w : bw;
+    best = key > best ? key : best;
+  }
+  const long long o = pair_out(a, pl, d, tt) + b;
+  if (best) a.out.put(o, (long long)(~(uint32_t)best), a.pval[(pl * a.nsplit + bw) * (long long)nb + b]);
+  else a.out.none(o);
 }
 
 // Columns: 16 columns f1 of one pair per workgroup; lane = 16 * t + s, so the
@@ -140,9 +131,9 @@ __device__ __forceinline__ void finish_cell(const BigArgs &a, long long np, long
 // cold templates: 63.2 us, of which reading alone takes 35 and writing alone
 // 23; with the walk 53.0 (195 MB, 3.7 TB/s; the same at three or four
 // workgroups per CU and with the data columns read ahead too).  At 4 waves per SIMD
-// the registers spill (59.9 us).
-template <class B>
-__global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu(3)))
+// the registers spill (59.9 us).  WALK false: one tile per workgroup (kColTiles).
+template <class B, bool WALK>
+__global__ void __launch_bounds__(16 * B::CT) __attribute__((amdgpu_waves_per_eu(WALK ? 3 : 4)))
 big_cols_kernel(BigArgs a, int np) {
   constexpr int N = B::N, ROW = B::ROW, CT = B::CT;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -156,17 +147,19 @@ big_cols_kernel(BigArgs a, int np) {
   // fall in distinct banks, its 4 row groups read the same words).
   cf *bt = reinterpret_cast<cf *>(smem) + 16 * B::COL_STRIDE;
   if (a.hint && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.hint = *a.list_count;
-  const int count = (int)min((long long)np, (a.list ? (long long)*a.list_count : (long long)a.nd * a.nt) - a.p0);
   int pl = (int)blockIdx.y;  // pair within the chunk
-  if (pl >= count) return;  // uniform; no barrier has run yet
+  int d = 0, tt = 0;
+  if (!big_pair(a, a.p0 + pl, d, tt)) return;  // uniform; no barrier has run yet
   const int f1 = blockIdx.x * 16 + s;
   cf wt{1.f, 0.f};
-  if constexpr (!B::RF) {
-    bt[17 * s + t] = big_root(a, 16 * f1 * t);  // u = t; 16 f1 t < n
-    wt = big_root(a, f1 * t);
-  }
+  auto closing_roots = [&]() {
+    if constexpr (!B::RF) {
+      bt[17 * s + t] = big_root(a, 16 * f1 * t);  // u = t; 16 f1 t < n
+      wt = big_root(a, f1 * t);
+    }
+  };
   cf w1{1.f, 0.f}, w4{1.f, 0.f};  // the column passes' twiddles depend on t only
-  if constexpr (B::ROWS == 256) {
+  if constexpr (WALK) {
     w1 = a.twCol[TwiddleLayout<256>::offset(1) + t];
     w4 = a.twCol[TwiddleLayout<256>::offset(1) + 16 + t];
   }
@@ -180,23 +173,10 @@ big_cols_kernel(BigArgs a, int np) {
     for (int u = 0; u < 16; u++)
       x[u] = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(r, voff, u * CT * ROW * (int)sizeof(cf), 0));
   };
-  int d = 0, tt = 0;
-  big_pair(a, a.p0 + pl, d, tt);
-  cf y[16];
-  load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
-  for (;;) {
-    cf v[16];
-    load(v, row_rsrc(a.data + (long long)d * a.data_stride));
-    const int next = pl + (int)gridDim.y;
-    const bool more = next < count;
-    if (more) big_pair(a, a.p0 + next, d, tt);
-#pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = cmul_conj(v[u], y[u]);
-    // the next pair's template is read while this one is transformed and stored
-    if (more) load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
-    __builtin_amdgcn_sched_barrier(0);
-    // the transform's barriers order the bt stores before the reads
-    if constexpr (B::ROWS == 256) {
+  // inverse transform of the columns and Y[k2][f1], k2 = t + CT u; its barriers
+  // order the bt stores before the reads
+  auto finish = [&](cf *v, int pl) {
+    if constexpr (WALK) {
       dft16(v);
       stockham_store<256, 16, 1>(v, t, xch);
       __syncthreads();
@@ -206,21 +186,51 @@ big_cols_kernel(BigArgs a, int np) {
 #pragma unroll
       for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
       dft16(v);
+      __builtin_amdgcn_sched_barrier(0);
     } else {
       inverse_fft<B::ROWS>(v, t, xch, a.twCol);
     }
-    __builtin_amdgcn_sched_barrier(0);
     const __amdgpu_buffer_rsrc_t ry = row_rsrc(a.scratch + (long long)pl * N);
-    const int yoff = (t * ROW + f1) * (int)sizeof(cf);  // Y[k2][f1], k2 = t + CT u
+    const int yoff = (t * ROW + f1) * (int)sizeof(cf);
 #pragma unroll
     for (int u = 0; u < 16; u++) {
       if constexpr (!B::RF) v[u] = cmul(v[u], cmul(wt, bt[17 * s + u]));
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v[u]), ry, yoff, u * CT * ROW * (int)sizeof(cf),
                                             0);
     }
-    if (!more) break;
-    pl = next;
-    __syncthreads();  // the exchange is read
+  };
+  if constexpr (!WALK) {
+    closing_roots();
+    const __amdgpu_buffer_rsrc_t rd = row_rsrc(a.data + (long long)d * a.data_stride);
+    const __amdgpu_buffer_rsrc_t rt = row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride);
+    cf v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int so = u * CT * ROW * (int)sizeof(cf);
+      const cf x = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rd, voff, so, 0));
+      const cf y = __builtin_bit_cast(cf, __builtin_amdgcn_raw_buffer_load_b64(rt, voff, so, 0));
+      v[u] = cmul_conj(x, y);
+    }
+    finish(v, pl);
+  } else {
+    cf y[16];
+    load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
+    closing_roots();
+    for (;;) {
+      cf v[16];
+      load(v, row_rsrc(a.data + (long long)d * a.data_stride));
+      const int next = pl + (int)gridDim.y;
+      const bool more = next < np && big_pair(a, a.p0 + next, d, tt);
+#pragma unroll
+      for (int u = 0; u < 16; u++) v[u] = cmul_conj(v[u], y[u]);
+      // the next pair's template is read while this one is transformed and stored
+      if (more) load(y, row_rsrc(a.tmpl + (long long)tt * a.tmpl_stride));
+      __builtin_amdgcn_sched_barrier(0);
+      finish(v, pl);
+      if (!more) break;
+      pl = next;
+      __syncthreads();  // the exchange is read
+    }
   }
 }
 
@@ -252,8 +262,8 @@ __device__ __forceinline__ void closing_passes(cf *v, int t, int k, cf *xch, con
 // Rows: nsplit workgroups per pair (workgroup = pair * nsplit + part), each
 // walking its share of the rows k2, SLOTS rows at a time.  With one part
 // the table is the result; with several, each part leaves its (key, value)
-// table and merge_cell keeps the largest key per bin: in the pair's last part
-// or, for large tables, by finish_cell in the next chunk's rows launch or in
+// table and the largest key per bin is kept: by the pair's last part (RF > 0
+// and small tables), else by finish_cell in the next chunk's rows launch or in
 // big_rows_finish_kernel after the last chunk.
 template <class B>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
@@ -370,13 +380,40 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
   const long long o = pair_out(a, pl, d, tt);
   if (a.nsplit > 1) {
     const long long po = (pl * a.nsplit + part) * (long long)nb;
+    if (!B::RF || !a.done) {
+      for (int b = threadIdx.x; b < nb; b += 256) {
+        const uint64_t key = bkey[b];
+        a.pkey[po + b] = key;
+        a.pval[po + b] = key ? bval[b] : cf{0.f, 0.f};
+      }
+      return;
+    }
     for (int b = threadIdx.x; b < nb; b += 256) {
       const uint64_t key = bkey[b];
       part_put(a.pkey + po + b, key);
       part_put((uint64_t *)a.pval + po + b, key ? __builtin_bit_cast(uint64_t, bval[b]) : 0ull);
     }
-    if (a.done && part_is_last(a.done + pl, a.nsplit, *reinterpret_cast<int *>(smem)))
-      for (int b = threadIdx.x; b < nb; b += 256) merge_cell(a, pl, b, o + b);
+    if (!part_is_last(a.done + pl, a.nsplit, *reinterpret_cast<int *>(smem))) return;
+    // the others' keys into this part's own table, all loads at once; then a
+    // bin's value from the part that holds its winning lag's row
+    const uint64_t *keys = a.pkey + pl * a.nsplit * (long long)nb;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < a.nsplit * nb; i += 256) {
+      const uint64_t key = part_get(keys + i);
+      if (key) atomicMax((unsigned long long *)&bkey[i % nb], (unsigned long long)key);
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < nb; b += 256) {
+      const uint64_t key = bkey[b];
+      if (!key) {
+        a.out.none(o + b);
+        continue;
+      }
+      const uint32_t k = ~(uint32_t)key;
+      const int w = (int)(k % ROWS) / SLOTS * a.nsplit / G;  // both powers of two
+      const uint64_t *vals = (const uint64_t *)a.pval + (pl * a.nsplit + w) * (long long)nb;
+      a.out.put(o + b, (long long)k, __builtin_bit_cast(cf, part_get(vals + b)));
+    }
     return;
   }
   for (int b = threadIdx.x; b < nb; b += 256) {
@@ -403,10 +440,17 @@ __global__ void roots_kernel(cf *out, int L, int period) {
 }
 
 constexpr size_t kLds = 160 * 1024;
-// Table entries that a pair's last part merges: n = 262144, 2 x 31 pairs, 64 bins x
-// 16 parts 104.0 us a call against 105.8 with finish_cell, 512 x 16 110.7
-// against 116.2; 131072, 2 x 10, 2048 x 32: 67.5 against 56.8.  One pair: 35.4 and 36.4.
+// n = 32768 and 65536, whose calls are small here: a pair's last part merges up to so
+// many table entries (1 x 4 pairs at 65536 32.8 us a call against 34.0 with a finish launch,
+// 2 x 10 at 32768 32.6 against 34.0).  Longer rows keep the finish launch, most
+// of which run inside the next chunk's rows launch: merging there took 2 x 31
+// pairs at 262144 from 104.8 to 102.7, but 1 x 20 from 53.7 to 57.8 and 4 x 64
+// from 321 to 330.
 constexpr size_t kMergeCells = 8192;
+// Walking pairs pays from a good third more tiles than a launch has resident (us a
+// call, walk / one tile each; tiles): 1280 49.5 / 48.2 and 53.9 / 53.7, 1440 57.6 /
+// 60.2, 1536 66.7 / 67.5, 1792 67.7 / 69.0, 3968 104.8 / 111.
+constexpr int kColTiles = 1400;
 constexpr int kColGrid = 1024;  // columns workgroups per launch: four per CU, of which three are resident at a time
 
 template <class B>
@@ -455,7 +499,8 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
   a.inv_bs = 1.0f / (float)r.binsize;
   const size_t nb_total = (r.we - r.ws + r.binsize - 1) / r.binsize;
   const size_t maxb = rows_max_bins<B>();
-  if (!lds_limit((const void *)big_cols_kernel<B>, c->dev, lds_cols) ||
+  if (!lds_limit((const void *)big_cols_kernel<B, false>, c->dev, lds_cols) ||
+      !lds_limit((const void *)big_cols_kernel<B, !B::RF>, c->dev, lds_cols) ||
       !lds_limit((const void *)big_rows_kernel<B>, c->dev, kLds))
     return -1;
   // rows workgroups per pair: enough for about 1024 workgroups per launch (at
@@ -479,11 +524,11 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
     pval2 = (cf *)c->scratch("big_part_val", 2 * part_cells * sizeof(cf));
     if (!pkey2 || !pval2) return -1;
   }
-  // a pair's last part merges the tables where that is little work for one
-  // workgroup; else the finish of a chunk runs in the next rows launch when the
-  // window is one piece (one rows launch per chunk), and after each rows launch when not
+  // where the pairs' last parts do not merge the tables, the finish of a chunk
+  // runs in the next rows launch when the window is one piece (one rows launch
+  // per chunk), and after each rows launch when not
   a.done = nullptr;
-  if (nsplit > 1) {
+  if (B::RF && nsplit > 1) {
     a.done = c->part_counters((size_t)chunk);  // in any case: a later, captured call may have fewer bins
     if (!a.done) return -1;
     if (nb_piece * nsplit > kMergeCells) a.done = nullptr;
@@ -501,9 +546,15 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
       a.pkey = pkey2 + (ci & 1) * part_cells;
       a.pval = pval2 + (ci & 1) * part_cells;
     }
-    const unsigned walkers = (unsigned)std::min<long long>(np, kColGrid / (B::ROW / 16));
-    hipLaunchKernelGGL(big_cols_kernel<B>, dim3(B::ROW / 16, walkers), dim3(16 * B::CT), lds_cols, c->stream, a,
-                       (int)np);
+    // the first with one tile per workgroup
+    const long long tiles = np * (B::ROW / 16);
+    if (!B::RF && tiles > kColTiles) {
+      hipLaunchKernelGGL((big_cols_kernel<B, !B::RF>), dim3(B::ROW / 16, kColGrid / (B::ROW / 16)), dim3(16 * B::CT),
+                         lds_cols, c->stream, a, (int)np);
+    } else {
+      hipLaunchKernelGGL((big_cols_kernel<B, false>), dim3(B::ROW / 16, (unsigned)np), dim3(16 * B::CT), lds_cols,
+                         c->stream, a, (int)np);
+    }
     if (!hip_ok(hipGetLastError(), "big_cols_kernel")) return -1;
     a.hint = nullptr;
     for (size_t b0 = 0; b0 < nb_total; b0 += maxb) {
