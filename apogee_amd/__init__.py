@@ -32,7 +32,7 @@ PEAK_DTYPE = np.dtype([("index", "<i8"), ("value", "<c8")])
 _GPU_SIZES = frozenset((64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384,
                         32768, 65536))
 #: Lengths this build adds beyond the reference's GPU set (its CPU engine's
-#: larger power-of-two lengths), carried by the same four-step split.
+#: larger power-of-two lengths), carried by a four-step split.
 _LARGE_SIZES = frozenset((131072, 262144, 524288, 1048576))
 
 __all__ = ["MatchedFilter", "HierarchicalFilter", "RefineQueue", "PEAK_DTYPE", "devices",

@@ -3,10 +3,10 @@
 Tunables (each a key of the library's tuning interface):
 
 * ``flat`` -- ``dpw``: data rows each workgroup of the tiled flat kernel
-  walks while its template stays in registers (more rows: fewer template
-  reads and fewer, longer workgroups; fewer rows: more workgroups in flight);
-* ``big`` -- ``big_chunk_mb``: for the four-step lengths (n >= 32768), the
-  pairs whose n-point intermediate is held at once (column launch, then row
+  walks (more rows: fewer, longer workgroups; fewer rows: more workgroups in
+  flight; one by default, and a tuned tile only where it leaves 1024 of them);
+* ``big`` -- ``big_chunk_mb``: for the two-kernel lengths (n >= 131072, and
+  32768 and 65536 with few pairs), the pairs whose n-point intermediate is held at once (column launch, then row
   launch, per chunk): larger chunks mean fewer, fuller launches until the
   intermediate no longer stays in the memory-side cache between the two;
 * ``hier`` -- ``refine_grid``: workgroups of the list-driven refine launch,

@@ -346,7 +346,7 @@ long mfh_hier_run_series_rec(mfh_ctx *ctx, const void *series_c64, size_t nserie
  * read from LDS), "coarse_fuse" (0/1, on by default: at n = 4096 with one
  * bin and the constants in LDS, the screen's workgroups refine their own
  * survivors in the same launch), "big_chunk_mb" (scratch
- * per column / row launch pair at n >= 32768), "wide" (n = 8192 ... 65536, one
+ * per column / row launch pair of the two-kernel path), "wide" (n = 8192 ... 65536, one
  * workgroup per pair or half of one: 0 = by the pair count, 1 = always,
  * 2 = never; results are the same), "totals" (1 by default; 0: runs with host
  * results return 0 instead of the number of reported bins unless per-pair
