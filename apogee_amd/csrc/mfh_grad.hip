@@ -361,13 +361,18 @@ __global__ void __launch_bounds__(256) peak_value_kernel(const cf *__restrict__ 
 
 }  // namespace
 
+// Elements of partial sums behind the root tables (n >= 1024): splits x rows x n
+// is at most 256 workgroups' tiles of 512 whatever the call, so that one call
+// of a context leaves all that any later, captured one needs.
+constexpr size_t kGradPart = 256 * 512;
+
 static const cf *unit_circle(Ctx *c) {
   char name[32];
   snprintf(name, sizeof name, "circle%zu", c->n);
   auto it = c->bufs.find(name);
   if (it != c->bufs.end() && it->second.p) return (const cf *)it->second.p;
   const int nh = c->n >= 256 ? (int)(c->n / 256) : 1;
-  cf *r = (cf *)c->scratch(name, (size_t)(nh + 256) * sizeof(cf));
+  cf *r = (cf *)c->scratch(name, ((size_t)(nh + 256) + (c->n >= 1024 ? kGradPart : 0)) * sizeof(cf));
   if (!r) return nullptr;
   hipLaunchKernelGGL(circle_tables_kernel, dim3((unsigned)((nh + 256 + 255) / 256)), dim3(256), 0, c->stream, r,
                      (int)c->n);
@@ -392,13 +397,7 @@ static int launch_grad_mfma(Ctx *c, const cf *other, long long other_stride, int
   splits = (int)std::max<long long>(1, std::min<long long>(splits, (long long)nother * nb / 64));
   const int per = (nother + splits - 1) / splits;
   splits = (nother + per - 1) / per;
-  cf *dst = out;
-  if (splits > 1) {
-    // splits * rows * n <= 256 * 512 elements whatever the call: one size for
-    // all, so that a later call never replaces the buffer
-    dst = (cf *)c->scratch("grad_part", 256 * 512 * sizeof(cf));
-    if (!dst) return -1;
-  }
+  cf *dst = splits > 1 ? const_cast<cf *>(roots) + n / 256 + 256 : out;  // kGradPart
   hipLaunchKernelGGL(peak_grad_mfma_kernel<TEMPL>, dim3(tiles, rows, splits), dim3(512), 0, c->stream, other,
                      other_stride, nother, per, idx, gval, nt, nb, roots, n, dst, (long long)n);
   if (!hip_ok(hipGetLastError(), "peak_grad_mfma_kernel")) return -1;
