@@ -640,11 +640,15 @@ constexpr size_t wide_lds() {
 
 using WideKernel = void (*)(WideArgs);
 
-// The kernel for a launch of nb bins and this seed, its LDS limit raised.
+// The kernel for a launch of nb bins and this seed, its LDS limit raised.  List
+// launches take the rolled selection without a threshold too: beside the list's own
+// state the unrolled one spills (a mixed queue without thresholds: 812 us a run
+// against 692; 757 before this path).
 template <class W, bool LIST>
 WideKernel wide_pick(Ctx *c, size_t nb, bool dense) {
-  const WideKernel k = nb == 1 ? (dense ? wide_kernel<W, true, true, LIST> : wide_kernel<W, true, false, LIST>)
-                               : (dense ? wide_kernel<W, false, true, LIST> : wide_kernel<W, false, false, LIST>);
+  const WideKernel k =
+      nb == 1 ? (dense ? wide_kernel<W, true, !LIST, LIST> : wide_kernel<W, true, false, LIST>)
+              : (dense ? wide_kernel<W, false, !LIST, LIST> : wide_kernel<W, false, false, LIST>);
   return lds_limit((const void *)k, c->dev, wide_lds<W>()) ? k : nullptr;
 }
 
