@@ -111,10 +111,27 @@ __global__ void gate_kernel(const int64_t *cidx, const cf *cval, int nd, int nt,
 // pairs leave in longer runs (public run, 16 x 1024, one row with a signal /
 // noise: 4 x 4 47.6 / 42.1 us, 8 x 2 42.3 / 45.0, 16 x 1 48.6 / 53.5).
 constexpr int kGatePairs = 16;
-template <int FN, int MODE>
+
+// The screen that gate_refine_kernel runs itself (CM > 0): bands and window of
+// the FP32 screen's flat launch.
+struct GateScreen {
+  const cf *tmpl;     // coarse templates, CM apart
+  const cf *twiddle;  // of length CM
+  uint32_t ws, we;    // coarse window
+  float seed;
+};
+
+// CM = 64, 128 or 256: no screen launch before this one, which transforms its own
+// pairs' bands (one slot of CM / 16 lanes each, the flat kernel's arithmetic, so
+// the same decisions): one short transform per wave at the start, instead of a launch
+// of 7 us, the gap behind it and its results' way through memory.  Public
+// run, screen apart / inside, one row with a signal: 16 x 1024 band 64 53.8 / 50.5 us, 128
+// 44.0 / 41.8, 256 44.5 / 40.8; 16 x 4096 84.4 / 84.6, 76.3 / 68.7, 82.7 / 69.3;
+// 4 x 64 41.3 / 38.6, 37.9 / 35.2, 37.8 / 35.7.
+template <int FN, int MODE, int CM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, int rows, float thr, int *count, int *other,
-                   FlatArgs fa) {
+gate_refine_kernel(const int64_t *cidx, const cf *cval, GateScreen cs, int nd, int nt, int rows, float thr, int *count,
+                   int *other, FlatArgs fa) {
   using S = FlatShape<FN>;
   static_assert(S::WG == 256 && S::SLOTS == 1 && S::TPT == 256, "one transform per 256-thread workgroup");
   extern __shared__ __align__(16) unsigned char smem[];
@@ -123,13 +140,41 @@ gate_refine_kernel(const int64_t *cidx, const cf *cval, int nd, int nt, int rows
   const int lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *other = 0;  // the next call's counter
   const int nb = (int)fa.nb;
+  __shared__ int fired[CM ? kGatePairs : 1];
+  if constexpr (CM > 0) {
+    using C = FlatShape<CM>;
+    constexpr int TPT = C::TPT;
+    if ((int)threadIdx.x < kGatePairs * TPT) {  // whole waves
+      const int i = threadIdx.x / TPT, t = threadIdx.x % TPT;
+      const int d = blockIdx.y * rows + i % rows, tt = blockIdx.x * (kGatePairs / rows) + i / rows;
+      const bool inside = d < nd && tt < nt;
+      const cf *dp = fa.data + (inside ? d : 0) * fa.data_stride;
+      const cf *tp = cs.tmpl + (long long)(inside ? tt : 0) * CM;
+      cf wf[15], v[16];
+      first_twiddles<CM>(wf, t, cs.twiddle);
+#pragma unroll
+      for (int u = 0; u < 16; u++) v[u] = cmul_conj(dp[t + u * TPT], tp[t + u * TPT]);
+      inverse_fft<CM, true, true>(v, t, reinterpret_cast<cf *>(smem) + i * C::XSTRIDE, cs.twiddle, wf);
+      float m = 0.f;  // a NaN is never the larger operand of fmaxf
+#pragma unroll
+      for (int u = 0; u < 16; u++) {
+        const float m2 = __builtin_fmaf(v[u].x, v[u].x, v[u].y * v[u].y);
+        m = fmaxf(m, (uint32_t)(t + u * TPT) - cs.ws < cs.we - cs.ws ? m2 : 0.f);
+      }
+      const float best = __uint_as_float(group_umax<TPT>(__float_as_uint(m)));
+      if (t == 0) fired[i] = inside && best > cs.seed && sqrtf(best) >= thr;
+    }
+    __syncthreads();
+  }
   if (threadIdx.x < 64) {
     const int d = blockIdx.y * rows + lane % rows;
     const int tt = blockIdx.x * (kGatePairs / rows) + lane / rows;
     const bool inside = lane < kGatePairs && d < nd && tt < nt;
     const long long p = (long long)d * nt + tt;
     bool fire = false;
-    if (inside && cidx[p] >= 0) {
+    if constexpr (CM > 0) {
+      fire = inside && fired[lane % kGatePairs];
+    } else if (inside && cidx[p] >= 0) {
       const cf z = cval[p];
       const float m2 = __builtin_fmaf(z.x, z.x, z.y * z.y);
       fire = sqrtf(m2) >= thr;
@@ -248,24 +293,45 @@ static bool gate_refine_fits(const Ctx *c, size_t n, size_t nb, size_t ws, size_
   return c->coarse_fuse && n == 4096 && (nb == 1 || (ws % 64 == 0 && we % 64 == 0 && binsize % 64 == 0));
 }
 
-static int launch_gate_refine(Ctx *c, const int64_t *cidx, const cf *cval, int nd, int nt, float thr, int *count,
-                              int *other, const FlatRun &rr) {
+// Whether the launch above screens too: bands whose 16 transforms fill a
+// workgroup at most (at 512 they would take two turns, in more LDS than the refine).
+static bool gate_screens(size_t band) { return band == 64 || band == 128 || band == 256; }
+
+// `cr`: the screen's flat launch, which has run unless gate_screens(band).
+static int launch_gate_refine(Ctx *c, size_t band, const FlatRun &cr, const int64_t *cidx, const cf *cval, int nd,
+                              int nt, float thr, int *count, int *other, const FlatRun &rr) {
   constexpr int FN = 4096;
   FlatArgs fa;
   if (flat_fill_args(c, FN, rr, fa) < 0) return -1;
   const int nb = (int)fa.nb;
   if (!gate_refine_fits(c, FN, nb, fa.ws, fa.we, fa.binsize))
     return fail("the one-launch gate and refine does not apply here");
-  using Kern = decltype(&gate_refine_kernel<FN, kOneBin>);
-  const Kern kern = nb == 1 ? gate_refine_kernel<FN, kOneBin> : gate_refine_kernel<FN, kAligned>;
+  using Kern = decltype(&gate_refine_kernel<FN, kOneBin, 0>);
+  Kern kern = nb == 1 ? gate_refine_kernel<FN, kOneBin, 0> : gate_refine_kernel<FN, kAligned, 0>;
+  GateScreen cs{};
+  size_t screen_lds = 0;
+  if (gate_screens(band)) {
+    if (band == 64) kern = nb == 1 ? gate_refine_kernel<FN, kOneBin, 64> : gate_refine_kernel<FN, kAligned, 64>;
+    if (band == 128) kern = nb == 1 ? gate_refine_kernel<FN, kOneBin, 128> : gate_refine_kernel<FN, kAligned, 128>;
+    if (band == 256) kern = nb == 1 ? gate_refine_kernel<FN, kOneBin, 256> : gate_refine_kernel<FN, kAligned, 256>;
+    cs.tmpl = cr.tmpl;
+    cs.twiddle = c->twiddles(band);
+    if (!cs.twiddle) return -1;
+    cs.ws = (uint32_t)cr.ws;
+    cs.we = (uint32_t)cr.we;
+    cs.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
+    const size_t slot = band == 64 ? FlatShape<64>::XSTRIDE : band == 128 ? FlatShape<128>::XSTRIDE : FlatShape<256>::XSTRIDE;
+    screen_lds = kGatePairs * slot * sizeof(cf);
+  }
   const int rows = c->many_refined((long long)nd * nt) ? 8 : 4;
   const int templates = kGatePairs / rows;
   const dim3 grid((unsigned)((nt + templates - 1) / templates), (unsigned)((nd + rows - 1) / rows));
-  if (grid.y > 65535) return fail("too many data rows per launch (%d)", nd);
-  const size_t smem = (size_t)FlatShape<FN>::XSTRIDE * sizeof(cf) + 2 * (size_t)nb * sizeof(uint64_t);
+  if ((nd + 3) / 4 > 65535) return fail("too many data rows per launch (%d)", nd);  // whichever tile
+  const size_t smem =
+      std::max(screen_lds, (size_t)FlatShape<FN>::XSTRIDE * sizeof(cf) + 2 * (size_t)nb * sizeof(uint64_t));
   if (!lds_limit((const void *)kern, c->dev, smem)) return -1;
   Ctx::ProfScope ps(c, "refine");
-  hipLaunchKernelGGL(kern, grid, dim3(256), smem, c->stream, cidx, cval, nd, nt, rows, thr, count, other, fa);
+  hipLaunchKernelGGL(kern, grid, dim3(256), smem, c->stream, cidx, cval, cs, nd, nt, rows, thr, count, other, fa);
   return hip_ok(hipGetLastError(), "gate_refine_kernel") ? 0 : -1;
 }
 
@@ -371,12 +437,14 @@ int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float thres
   cr.prof_name = "coarse";
   cr.zero = count;  // the coarse launch clears the survivor counter
   if (!mfma) {
-    if (launch_flat(c, m, cr) < 0) return -1;
-    if (gate_refine_fits(c, n, nb, ws, we, binsize)) {
-      // the gate and the refine in one launch; the screen above cleared this
-      // call's counter, the launch clears the next call's
+    const bool one = gate_refine_fits(c, n, nb, ws, we, binsize);
+    if (!(one && gate_screens(m)) && launch_flat(c, m, cr) < 0) return -1;
+    if (one) {
+      // the gate and the refine in one launch, short bands' screen with them;
+      // this call's counter is clear (by the previous call, and by the screen
+      // above where it ran), the launch clears the next call's
       const FlatRun rr = refine_base(c, drows, t0, nd, nt, binsize, threshold, ws, we, out);
-      if (launch_gate_refine(c, cidx, cval, nd, nt, coarse_thr, count, other, rr) < 0) return -1;
+      if (launch_gate_refine(c, m, cr, cidx, cval, nd, nt, coarse_thr, count, other, rr) < 0) return -1;
       if (!c->capturing && !hs) c->hier_parity ^= 1;
       return deliver_refined(c, count, refined);
     }

@@ -344,8 +344,9 @@ long mfh_hier_run_series_rec(mfh_ctx *ctx, const void *series_c64, size_t nserie
  * (templates per wave of the matrix-core coarse screen, 1..64), "coarse_rpw"
  * (its data rows per wave, 1 or 2), "coarse_lds" (0/1: its DFT constants
  * read from LDS), "coarse_fuse" (0/1, on by default: at n = 4096 with one
- * bin and the constants in LDS, the screen's workgroups refine their own
- * survivors in the same launch), "big_chunk_mb" (scratch
+ * bin and the constants in LDS, the matrix-core screen's workgroups refine their own
+ * survivors in the same launch; with the FP32 screen, gate and refine share a
+ * launch, which at bands up to 256 also screens), "big_chunk_mb" (scratch
  * per column / row launch pair of the two-kernel path), "wide" (n = 8192 ... 65536, one
  * workgroup per pair or half of one: 0 = by the pair count, 1 = always,
  * 2 = never; results are the same), "totals" (1 by default; 0: runs with host

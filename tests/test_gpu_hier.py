@@ -105,6 +105,33 @@ def test_survivors_beyond_the_column_workgroups(gpu_device):
     assert fired.any(axis=-1).sum() > 32
 
 
+@pytest.mark.parametrize("nd,nt", [(1, 1), (5, 7), (9, 30)])
+@pytest.mark.parametrize("band", [64, 128, 256])
+def test_screen_inside_the_refine_launch(band, nd, nt, gpu_device):
+    """Short bands screened by the gate-and-refine launch: the same survivors and
+    results as with launches of their own, for whole and partial tiles, windows, bins,
+    and rows that hold a NaN or nothing."""
+    n = 4096
+    power, D, H = loud_case(n, nd, nt, seed=band + nt, snr=9.0)
+    D = np.array(D)
+    if nd > 2:
+        D[1, 3] = np.nan
+        D[2] = 0
+    _, hier = build(n, nd, nt, power, band=band)
+    hier.set_data(D)
+    hier.set_templates(H)
+    for binsize, threshold, window in [(n, 5.5, None), (n, 3.0, (100, 3000)), (512, 4.0, None), (64, 4.5, (64, 2048))]:
+        kw = {} if window is None else {"window": window}
+        out = []
+        for fuse in (0, 1, 1):
+            hier._gpu.set_tuning("coarse_fuse", fuse)
+            out.append((hier.run(binsize=binsize, threshold=threshold, **kw), hier._gpu.last_refinements))
+        for got, refined in out[1:]:
+            np.testing.assert_array_equal(got["index"], out[0][0]["index"])
+            np.testing.assert_array_equal(got["value"], out[0][0]["value"])
+            assert refined == out[0][1]
+
+
 @pytest.mark.parametrize("threshold", [3.0, 5.5, 8.0, 20.0])
 def test_thresholds(threshold, gpu_device):
     a, b, _ = run_both(4096, 2, 4, 512, threshold, None)
