@@ -8,8 +8,8 @@
 // of the one-workgroup transform (mfh_wide.hip), the first two in kernel A
 // (256 columns of 16 RF points), the last two in kernel B (16 RF rows of 256
 // points), with the same arithmetic and so the same bits.  Spread over many
-// workgroups, one pair takes 14 us instead of 33 at n = 65536; from about
-// a hundred pairs on the scratch round trip costs more than it gives.
+// workgroups, one pair takes 14 us instead of 33 at n = 65536; from about 30 pairs
+// on the scratch round trip costs more than it gives.
 // Kernel A forms the product D*conj(T) on load, runs 256-point inverse FFTs
 // over 16 columns per workgroup and writes Y k2-major to scratch (each
 // 16-lane group writes 128 contiguous bytes).  Kernel B gives each pair a few

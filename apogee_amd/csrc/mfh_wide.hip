@@ -46,11 +46,11 @@ namespace {
 
 // From how many pairs a call takes this path, by length 8192 ... 65536.  Below,
 // more threads per pair win: at 8192 and 16384 one workgroup per CU of the
-// 16-point kernel (256 pairs: 7.6 against 9.6 us and 12.0 against 12.1; 384
-// pairs: 10.7 against 10.2 and 21.5 against 16.4), at 32768 and 65536 the
-// two-kernel path (16 pairs: 14.5 against 15.9 us, 32: 17.6 against 16.1;
-// 32 pairs: 23.7 against 25.9, 64: 27.7 against 25.5).
-constexpr long long kWideMinPairs[4] = {257, 257, 24, 56};
+// 16-point kernel (256 pairs: 8.2 against 9.4 us and 12.1 against 12.4; 384
+// pairs: 11.5 against 10.8 and 22.1 against 17.6), at 32768 and 65536 the
+// two-kernel path (24 pairs: 14.3 against 14.8 us, 32: 16.0 against 15.0;
+// 32 pairs: 24.6 against 24.4, 48: 28.0 against 24.4).
+constexpr long long kWideMinPairs[4] = {257, 257, 28, 32};
 
 struct WideArgs {
   FlatArgs f;              // rows, window, bins, outputs, list
