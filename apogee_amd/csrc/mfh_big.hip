@@ -454,14 +454,80 @@ constexpr int kColTiles = 1400;
 constexpr int kColGrid = 1024;  // columns workgroups per launch: four per CU, of which three are resident at a time
 
 template <class B>
+constexpr size_t big_cols_lds() {
+  return (16 * B::COL_STRIDE + 16 * 17) * sizeof(cf);
+}
+
+template <class B>
 size_t rows_max_bins() {
   using S = FlatShape<B::ROW>;
   return (kLds - (size_t)S::SLOTS * S::XSTRIDE * sizeof(cf)) / (sizeof(uint64_t) + sizeof(cf));
 }
 
+// What launches of up to `total` pairs with nb_total bins run in: pairs per chunk,
+// rows workgroups per pair, and the buffers, which `a` and `b` then point to.
+struct BigBuffers {
+  long long chunk;
+  size_t part_cells;
+  uint64_t *pkey2 = nullptr;
+  cf *pval2 = nullptr;
+};
+
+template <class B>
+int big_buffers(Ctx *c, long long total, size_t nb_total, BigArgs &a, BigBuffers &b) {
+  constexpr int N = B::N;
+  using S = FlatShape<B::ROW>;
+  a.twCol = c->twiddles(B::ROWS);
+  a.twRow = c->twiddles(B::RF ? N : B::ROW);
+  if (!a.twCol || !a.twRow) return -1;
+  a.rootH = a.rootL = nullptr;
+  if (!B::RF) {
+    const cf *roots = big_roots(c, B::ROW);
+    if (!roots) return -1;
+    a.rootH = roots;
+    a.rootL = roots + B::ROW;
+  }
+  // scratch in chunks of pairs: at most c->big_chunk_bytes of intermediate data
+  b.chunk = std::max<long long>(1, std::min<long long>(total, c->big_chunk_bytes / ((long long)N * 8)));
+  a.scratch = (cf *)c->scratch("big_scratch", (size_t)b.chunk * N * sizeof(cf));
+  if (!a.scratch) return -1;
+  if (!lds_limit((const void *)big_cols_kernel<B, false>, c->dev, big_cols_lds<B>()) ||
+      !lds_limit((const void *)big_cols_kernel<B, !B::RF>, c->dev, big_cols_lds<B>()) ||
+      !lds_limit((const void *)big_rows_kernel<B>, c->dev, kLds))
+    return -1;
+  // rows workgroups per pair: enough for about 1024 workgroups per launch (at
+  // least 8, at most one per row group), as long as the per-part tables stay
+  // within 64 MiB
+  constexpr int G = B::ROWS / S::SLOTS;
+  const size_t nb_piece = std::min(rows_max_bins<B>(), nb_total);
+  int nsplit = (int)std::min<long long>(G, std::max<long long>(8, (1024 + b.chunk - 1) / b.chunk));
+  nsplit = 1 << ilog2(nsplit);  // a power of two: parts split the row groups evenly
+  while (nsplit > 1 && (size_t)b.chunk * nsplit * nb_piece * 16 > (64ull << 20)) nsplit /= 2;
+  a.nsplit = nsplit;
+  a.pkey = nullptr;
+  a.pval = nullptr;
+  // part tables in two halves, by chunk parity: a rows launch writes one
+  // while its finishing blocks read the previous chunk's
+  b.part_cells = (size_t)b.chunk * nsplit * nb_piece;
+  if (nsplit > 1) {
+    b.pkey2 = (uint64_t *)c->scratch("big_part_key", 2 * b.part_cells * sizeof(uint64_t));
+    b.pval2 = (cf *)c->scratch("big_part_val", 2 * b.part_cells * sizeof(cf));
+    if (!b.pkey2 || !b.pval2) return -1;
+  }
+  // where the pairs' last parts do not merge the tables, the finish of a chunk
+  // runs in the next rows launch when the window is one piece (one rows launch
+  // per chunk), and after each rows launch when not
+  a.done = nullptr;
+  if (B::RF && nsplit > 1) {
+    a.done = c->part_counters((size_t)b.chunk);  // in any case: a later, captured call may have fewer bins
+    if (!a.done) return -1;
+    if (nb_piece * nsplit > kMergeCells) a.done = nullptr;
+  }
+  return 0;
+}
+
 template <class B>
 int launch_big_shape(Ctx *c, const FlatRun &r) {
-  constexpr int N = B::N;
   using S = FlatShape<B::ROW>;
   BigArgs a;
   a.data = r.data;
@@ -474,65 +540,19 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
   a.list_count = r.list_count;
   a.hint = r.list ? r.hint : nullptr;
   a.list_ooff = r.list_ooff;
-  a.twCol = c->twiddles(B::ROWS);
-  a.twRow = c->twiddles(B::RF ? N : B::ROW);
-  if (!a.twCol || !a.twRow) return -1;
-  a.rootH = a.rootL = nullptr;
-  if (!B::RF) {
-    const cf *roots = big_roots(c, B::ROW);
-    if (!roots) return -1;
-    a.rootH = roots;
-    a.rootL = roots + B::ROW;
-  }
-  const long long total = r.list ? (long long)r.list_cap : (long long)r.nd * r.nt;
-  // scratch in chunks of pairs: at most c->big_chunk_bytes of intermediate data
-  const long long chunk = std::max<long long>(1, std::min<long long>(total, c->big_chunk_bytes / ((long long)N * 8)));
-  cf *scr = (cf *)c->scratch("big_scratch", (size_t)chunk * N * sizeof(cf));
-  if (!scr) return -1;
-  a.scratch = scr;
-  const size_t lds_cols = (16 * B::COL_STRIDE + 16 * 17) * sizeof(cf);
   const float thr = r.threshold;
   a.seed = thr > 0.f ? (float)((double)thr * (double)thr) : 0.f;
   a.binsize = (uint32_t)r.binsize;
   const bool pow2 = (r.binsize & (r.binsize - 1)) == 0;
   a.bshift = pow2 ? ilog2((int)r.binsize) : -1;
   a.inv_bs = 1.0f / (float)r.binsize;
+  const long long total = r.list ? (long long)r.list_cap : (long long)r.nd * r.nt;
   const size_t nb_total = (r.we - r.ws + r.binsize - 1) / r.binsize;
   const size_t maxb = rows_max_bins<B>();
-  if (!lds_limit((const void *)big_cols_kernel<B, false>, c->dev, lds_cols) ||
-      !lds_limit((const void *)big_cols_kernel<B, !B::RF>, c->dev, lds_cols) ||
-      !lds_limit((const void *)big_rows_kernel<B>, c->dev, kLds))
-    return -1;
-  // rows workgroups per pair: enough for about 1024 workgroups per launch (at
-  // least 8, at most one per row group), as long as the per-part tables stay
-  // within 64 MiB
-  constexpr int G = B::ROWS / S::SLOTS;
-  const size_t nb_piece = std::min(maxb, nb_total);
-  int nsplit = (int)std::min<long long>(G, std::max<long long>(8, (1024 + chunk - 1) / chunk));
-  nsplit = 1 << ilog2(nsplit);  // a power of two: parts split the row groups evenly
-  while (nsplit > 1 && (size_t)chunk * nsplit * nb_piece * 16 > (64ull << 20)) nsplit /= 2;
-  a.nsplit = nsplit;
-  a.pkey = nullptr;
-  a.pval = nullptr;
-  // part tables in two halves, by chunk parity: a rows launch writes one
-  // while its finishing blocks read the previous chunk's
-  const size_t part_cells = (size_t)chunk * nsplit * nb_piece;
-  uint64_t *pkey2 = nullptr;
-  cf *pval2 = nullptr;
-  if (nsplit > 1) {
-    pkey2 = (uint64_t *)c->scratch("big_part_key", 2 * part_cells * sizeof(uint64_t));
-    pval2 = (cf *)c->scratch("big_part_val", 2 * part_cells * sizeof(cf));
-    if (!pkey2 || !pval2) return -1;
-  }
-  // where the pairs' last parts do not merge the tables, the finish of a chunk
-  // runs in the next rows launch when the window is one piece (one rows launch
-  // per chunk), and after each rows launch when not
-  a.done = nullptr;
-  if (B::RF && nsplit > 1) {
-    a.done = c->part_counters((size_t)chunk);  // in any case: a later, captured call may have fewer bins
-    if (!a.done) return -1;
-    if (nb_piece * nsplit > kMergeCells) a.done = nullptr;
-  }
+  BigBuffers b;
+  if (big_buffers<B>(c, total, nb_total, a, b) < 0) return -1;
+  const long long chunk = b.chunk;
+  const int nsplit = a.nsplit;
   const bool fold = nsplit > 1 && nb_total <= maxb;
   BigArgs fin = a;
   long long fin_np = 0;
@@ -543,17 +563,17 @@ int launch_big_shape(Ctx *c, const FlatRun &r) {
     const long long np = std::min(chunk, total - p0);
     a.p0 = p0;
     if (nsplit > 1) {
-      a.pkey = pkey2 + (ci & 1) * part_cells;
-      a.pval = pval2 + (ci & 1) * part_cells;
+      a.pkey = b.pkey2 + (ci & 1) * b.part_cells;
+      a.pval = b.pval2 + (ci & 1) * b.part_cells;
     }
     // the first with one tile per workgroup
     const long long tiles = np * (B::ROW / 16);
     if (!B::RF && tiles > kColTiles) {
       hipLaunchKernelGGL((big_cols_kernel<B, !B::RF>), dim3(B::ROW / 16, kColGrid / (B::ROW / 16)), dim3(16 * B::CT),
-                         lds_cols, c->stream, a, (int)np);
+                         big_cols_lds<B>(), c->stream, a, (int)np);
     } else {
-      hipLaunchKernelGGL((big_cols_kernel<B, false>), dim3(B::ROW / 16, (unsigned)np), dim3(16 * B::CT), lds_cols,
-                         c->stream, a, (int)np);
+      hipLaunchKernelGGL((big_cols_kernel<B, false>), dim3(B::ROW / 16, (unsigned)np), dim3(16 * B::CT),
+                         big_cols_lds<B>(), c->stream, a, (int)np);
     }
     if (!hip_ok(hipGetLastError(), "big_cols_kernel")) return -1;
     a.hint = nullptr;
@@ -606,6 +626,22 @@ const cf *big_roots(Ctx *c, int n1) {
     c->big_roots_ready[ilog2(n1)] = true;
   }
   return roots;
+}
+
+template <class B>
+static int reserve_shape(Ctx *c, long long pairs, size_t nb) {
+  BigArgs a;
+  BigBuffers b;
+  return big_buffers<B>(c, pairs, nb, a, b);
+}
+
+int big_reserve(Ctx *c, size_t n, const FlatRun &r, long long pairs) {
+  const size_t nb = (r.we - r.ws + r.binsize - 1) / r.binsize;
+  switch (n) {
+    case 32768: return reserve_shape<BigShape<0, 8>>(c, pairs, nb);
+    case 65536: return reserve_shape<BigShape<0, 16>>(c, pairs, nb);
+    default: return 0;
+  }
 }
 
 int launch_big(Ctx *c, size_t n, const FlatRun &r) {

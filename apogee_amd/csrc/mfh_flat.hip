@@ -246,6 +246,9 @@ size_t flat_row_window_bins(const Ctx *c, size_t n, const FlatRun &r) {
   }
 }
 
+// Lengths that either the one-workgroup or the two-kernel path serves.
+static bool two_paths(size_t n) { return n == 32768 || n == 65536; }
+
 int launch_flat(Ctx *c, size_t n, const FlatRun &r) {
   if (r.binsize < 1) return fail("binsize must be >= 1");
   size_t we = std::min(r.we, n);
@@ -253,9 +256,20 @@ int launch_flat(Ctx *c, size_t n, const FlatRun &r) {
   FlatRun q = r;
   q.we = we;
   hipSetDevice(c->dev);
-  // a list may take either path from one call to the next (wide_takes)
-  if (r.list && r.hint && !c->capturing && !c->no_alloc && wide_reserve(c, n, q) < 0) return -1;
-  if (wide_takes(c, n, q)) return launch_wide(c, n, q);
+  // A list may take either path from one call to the next (wide_takes), and an
+  // allocation-free call over part of the bank the one that this call does
+  // not: both find their buffers after one call over the whole.
+  if (r.list && r.hint && !c->capturing && !c->no_alloc) {
+    const long long few = std::min<long long>(r.list_cap, wide_min_pairs(n) - 1);
+    if (wide_reserve(c, n, q) < 0 || (few > 0 && big_reserve(c, n, q, few) < 0)) return -1;
+  }
+  bool wide = wide_takes(c, n, q);
+  // ... and with more bins than that call had, whichever of the two holds them
+  // (their results are the same bits)
+  if (r.list && c->no_alloc && two_paths(n) &&
+      (wide ? wide_reserve(c, n, q) : big_reserve(c, n, q, r.list_cap)) < 0)
+    wide = !wide;
+  if (wide) return launch_wide(c, n, q);
   switch (n) {
     case 64: return launch_len<64>(c, q);
     case 128: return launch_len<128>(c, q);

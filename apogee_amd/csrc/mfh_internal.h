@@ -222,11 +222,15 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
 // captured or allocation-free call of a list that may take either path).
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r);
 size_t wide_table_bins(size_t n);    // bins of one launch
-long long wide_min_pairs(size_t n);  // pairs from which an automatic run takes it
+long long wide_min_pairs(size_t n);  // pairs from which an automatic run takes it (0: no such length)
 int launch_wide(Ctx *c, size_t n, const FlatRun &r);
 int wide_reserve(Ctx *c, size_t n, const FlatRun &r);
 // The two-kernel flat filter for n >= 32768.
 int launch_big(Ctx *c, size_t n, const FlatRun &r);
+// Its buffers for up to `pairs` pairs of r made in advance (n = 32768 and 65536, where
+// an allocation-free call may take either path).  With Ctx::no_alloc set: < 0 if
+// they are not there.
+int big_reserve(Ctx *c, size_t n, const FlatRun &r, long long pairs);
 // Four-step root tables for n = n1 * 256: w_n1^h (h < n1) then w_n^l (l < 256),
 // FP64-generated once per context.
 const cf *big_roots(Ctx *c, int n1);

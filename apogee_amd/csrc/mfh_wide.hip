@@ -657,6 +657,11 @@ WideKernel wide_pick(Ctx *c, size_t nb, bool dense) {
 template <class W>
 int wide_tables(Ctx *c, WideArgs &wa, long long total, size_t nb, long long &chunk) {
   chunk = std::max<long long>(1, std::min<long long>(total, (64ll << 20) / ((long long)W::S * (long long)nb * 16)));
+  if (c->no_alloc) {  // the tables that are there, in more launches if need be
+    const auto have = c->bufs.find("wide_key");
+    const long long fit = have == c->bufs.end() ? 0 : (long long)(have->second.bytes / (W::S * nb * sizeof(uint64_t)));
+    if (fit > 0) chunk = std::min(chunk, fit);
+  }
   const size_t cells = (size_t)chunk * W::S * nb;
   wa.pkey = (uint64_t *)c->scratch("wide_key", cells * sizeof(uint64_t));
   wa.pval = (cf *)c->scratch("wide_val", cells * sizeof(cf));
@@ -740,7 +745,7 @@ size_t wide_table_bins(size_t n) {
   }
 }
 
-long long wide_min_pairs(size_t n) { return kWideMinPairs[ilog2((int)n) - 13]; }
+long long wide_min_pairs(size_t n) { return n < 8192 || n > 65536 ? 0 : kWideMinPairs[ilog2((int)n) - 13]; }
 
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   if (n < 8192 || n > 65536 || c->wide == 2) return false;
