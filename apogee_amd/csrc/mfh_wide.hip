@@ -653,8 +653,9 @@ WideKernel wide_pick(Ctx *c, size_t nb, bool dense) {
 }
 
 // The per-part tables of `total` pairs of nb bins, at most 64 MiB: `chunk` is
-// the pairs that they hold.
-template <class W>
+// the pairs that they hold.  A list launch has no part counters: they would have
+// to be of the largest chunk, which is that of the fewest bins.
+template <class W, bool LIST>
 int wide_tables(Ctx *c, WideArgs &wa, long long total, size_t nb, long long &chunk) {
   chunk = std::max<long long>(1, std::min<long long>(total, (64ll << 20) / ((long long)W::S * (long long)nb * 16)));
   if (c->no_alloc) {  // the tables that are there, in more launches if need be
@@ -665,8 +666,8 @@ int wide_tables(Ctx *c, WideArgs &wa, long long total, size_t nb, long long &chu
   const size_t cells = (size_t)chunk * W::S * nb;
   wa.pkey = (uint64_t *)c->scratch("wide_key", cells * sizeof(uint64_t));
   wa.pval = (cf *)c->scratch("wide_val", cells * sizeof(cf));
-  wa.done = c->part_counters((size_t)chunk);
-  return wa.pkey && wa.pval && wa.done ? 0 : -1;
+  wa.done = LIST ? nullptr : c->part_counters((size_t)chunk);
+  return wa.pkey && wa.pval && (LIST || wa.done) ? 0 : -1;
 }
 
 template <class W, bool LIST>
@@ -674,7 +675,7 @@ int wide_piece(Ctx *c, WideArgs &wa, long long total, size_t nb) {
   const WideKernel kern = wide_pick<W, LIST>(c, nb, wa.f.seed == 0.f);
   if (!kern) return -1;
   long long chunk = total;
-  if (W::S > 1 && wide_tables<W>(c, wa, total, nb, chunk) < 0) return -1;
+  if (W::S > 1 && wide_tables<W, LIST>(c, wa, total, nb, chunk) < 0) return -1;
   chunk = std::min(chunk, 1ll << 20);  // a launch holds fewer than 2^32 threads
   for (long long p0 = 0; p0 < total; p0 += chunk) {
     wa.p0 = p0;
@@ -730,7 +731,7 @@ int wide_ready(Ctx *c, const FlatRun &r) {
   const bool dense = !(r.threshold > 0.f);
   long long chunk;
   if (!wide_pick<W, true>(c, most, dense) || !wide_pick<W, true>(c, 1, dense)) return -1;
-  return W::S == 1 || wide_tables<W>(c, wa, (long long)r.list_cap, most, chunk) == 0 ? 0 : -1;
+  return W::S == 1 || wide_tables<W, true>(c, wa, (long long)r.list_cap, most, chunk) == 0 ? 0 : -1;
 }
 
 }  // namespace

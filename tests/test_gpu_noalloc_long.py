@@ -50,3 +50,20 @@ def test_part_of_the_bank_after_a_call_over_all_of_it(n):
         np.testing.assert_array_equal(v, av)
     finally:
         L.mfh_destroy(h)
+
+
+@pytest.mark.parametrize("n,nd,nt,binsize", [(65536, 16, 32, 8), (32768, 16, 40, 8)])
+def test_fewer_bins_than_the_call_that_built_the_buffers(n, nd, nt, binsize):
+    """The part tables hold fewer pairs at once the more bins a pair has: the
+    call with one bin, and so more pairs at once, finds its buffers too."""
+    L = lib()
+    h = make_ctx(L, n, nd, nt, 1024, 0, seed=n + 1)
+    try:
+        call(L, L.mfh_hier_peaks_async, h, 0, nd, 0, nt, binsize, 4.0, n, 3.8)
+        i, v = call(L, L.mfh_hier_peaks_noalloc, h, 0, nd, 0, nt, n, 4.0, n, 3.8)
+        ai, av = call(L, L.mfh_hier_peaks_async, h, 0, nd, 0, nt, n, 4.0, n, 3.8)
+        np.testing.assert_array_equal(i, ai)
+        np.testing.assert_array_equal(v, av)
+        assert (ai >= 0).any() and (ai < 0).any()
+    finally:
+        L.mfh_destroy(h)
