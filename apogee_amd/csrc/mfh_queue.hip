@@ -30,6 +30,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <initializer_list>
+#include <memory>
 #include <vector>
 
 #include "mfh_flat.h"
@@ -254,6 +256,8 @@ struct Queue {
     float threshold;
     long long ws, we;
     int first, count;  // entries in the device list
+    long long pairs;   // while planning: in all, and whether they go to a list
+    bool list;
   };
   std::vector<BigGroup> big;
   std::vector<long long> req_out;  // output offset per request
@@ -261,6 +265,43 @@ struct Queue {
   int grid_per_cu = 1;
   int grid_cap = 0;  // if > 0: at most this many persistent workgroups
   long prof_runs = 0;  // runs recorded while event timing is on
+};
+
+// Finds a request's group among those seen so far, in constant time: requests
+// with a window or threshold of their own are a group each (40000 of them plan
+// in 2 ms; a walk over the groups took 1.2 s).
+class GroupIndex {
+ public:
+  explicit GroupIndex(size_t requests) {
+    size_t cap = 16;
+    while (cap < 2 * requests) cap *= 2;
+    slot_.assign(cap, -1);
+  }
+  // the group like `like` (its list fields apart), appended if it is new
+  int find(std::vector<Queue::BigGroup> &groups, const Queue::BigGroup &like) {
+    uint32_t thr;
+    memcpy(&thr, &like.threshold, sizeof thr);
+    uint64_t h = (uint64_t)like.n;
+    for (const uint64_t x : {(uint64_t)like.binsize, (uint64_t)thr, (uint64_t)like.ws, (uint64_t)like.we}) {
+      h = (h ^ x) * 0x9e3779b97f4a7c15ull;
+      h ^= h >> 29;
+    }
+    for (size_t i = h & (slot_.size() - 1);; i = (i + 1) & (slot_.size() - 1)) {
+      int &g = slot_[i];
+      if (g < 0) {
+        g = (int)groups.size();
+        groups.push_back(like);
+        return g;
+      }
+      const Queue::BigGroup &G = groups[g];
+      if (G.n == like.n && G.binsize == like.binsize && !memcmp(&G.threshold, &like.threshold, sizeof thr) &&
+          G.ws == like.ws && G.we == like.we)
+        return g;
+    }
+  }
+
+ private:
+  std::vector<int> slot_;  // group by hash, at most half full
 };
 
 }  // namespace mfh
@@ -329,7 +370,8 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     return fail("null request array");
   std::vector<std::vector<QItem>> by_class(kQMaxLog2 + 1);
   std::vector<Queue::BigGroup> bigs;
-  std::vector<std::vector<std::pair<int2, long long>>> big_pairs;
+  std::unique_ptr<GroupIndex> index;
+  std::vector<int> group(nreq, -1);  // of each request that may go to a list launch
   q->req_out.assign(nreq, 0);
   q->req_nb.assign(nreq, 0);
   q->req_nc.assign(nreq, 0);
@@ -359,47 +401,48 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
       // long: one list entry per pair, grouped by launch parameters
       if (far)
         return fail("request %d: four-step spectra must start below pool element 2^31", r);
-      size_t g = 0;
-      for (; g < bigs.size(); g++) {
-        const auto &G = bigs[g];
-        if (G.n == (int)len && G.binsize == binsize[r] && !memcmp(&G.threshold, &thr, sizeof thr) &&
-            G.ws == ws[r] && G.we == we[r])
-          break;
-      }
-      if (g == bigs.size()) {
-        bigs.push_back({(int)len, (long long)binsize[r], thr, (long long)ws[r], (long long)we[r], 0, 0});
-        big_pairs.emplace_back();
-      }
-      for (int j = 0; j < ncand[r]; j++)
-        big_pairs[g].push_back({int2{(int)data_off[r], (int)(tmpl_off[r] + (long long)j * len)},
-                                nout + (long long)j * nb});
-    } else {
-      const QItem base = q_item(binsize[r], thr, ws[r], we[r], data_off[r]);
-      for (int j = 0; j < ncand[r]; j++) {
-        QItem it = base;
-        it.t_off = tmpl_off[r] + (long long)j * len;
-        it.o_off = nout + (long long)j * nb;
-        by_class[lg].push_back(it);
-      }
+      if (!index) index.reset(new GroupIndex((size_t)nreq));
+      group[r] = index->find(
+          bigs, {(int)len, (long long)binsize[r], thr, (long long)ws[r], (long long)we[r], 0, 0, 0, false});
+      bigs[group[r]].pairs += ncand[r];
     }
     nout += (long long)ncand[r] * nb;
     npairs += ncand[r];
   }
-  // groups of 8192 and 16384 too small for the one-workgroup path
-  for (size_t g = 0; g < bigs.size();) {
-    const auto G = bigs[g];
-    if (ilog2(G.n) > kQMaxLog2 || (long long)big_pairs[g].size() >= wide_min_pairs((size_t)G.n)) {
-      g++;
+  // the groups that get a list launch: not those of 8192 and 16384 too small for
+  // the one-workgroup path
+  long long listed = 0;
+  std::vector<int> bcount;
+  std::vector<Queue::BigGroup> lists;
+  for (auto &G : bigs) {
+    G.list = ilog2(G.n) > kQMaxLog2 || G.pairs >= wide_min_pairs((size_t)G.n);
+    if (!G.list) continue;
+    if (listed + G.pairs > INT32_MAX) return fail("too many pairs in one plan");
+    G.first = (int)listed;
+    G.count = 0;
+    listed += G.pairs;
+    bcount.push_back((int)G.pairs);
+    lists.push_back(G);
+    lists.back().count = (int)G.pairs;
+  }
+  std::vector<int2> blist((size_t)listed);
+  std::vector<long long> booff((size_t)listed);
+  for (int r = 0; r < nreq; r++) {
+    const long long len = n[r], nb = q->req_nb[r];
+    Queue::BigGroup *G = group[r] < 0 ? nullptr : &bigs[group[r]];
+    if (G && G->list) {
+      for (int j = 0; j < ncand[r]; j++, G->count++) {
+        blist[(size_t)G->first + G->count] = int2{(int)data_off[r], (int)(tmpl_off[r] + (long long)j * len)};
+        booff[(size_t)G->first + G->count] = q->req_out[r] + (long long)j * nb;
+      }
       continue;
     }
-    for (auto &e : big_pairs[g]) {
-      QItem it = q_item(G.binsize, G.threshold, G.ws, G.we, e.first.x);
-      it.t_off = e.first.y;
-      it.o_off = e.second;
-      by_class[ilog2(G.n)].push_back(it);
+    QItem it = q_item(binsize[r], threshold[r], ws[r], we[r], data_off[r]);
+    for (int j = 0; j < ncand[r]; j++) {
+      it.t_off = tmpl_off[r] + (long long)j * len;
+      it.o_off = q->req_out[r] + (long long)j * nb;
+      by_class[ilog2((int)len)].push_back(it);
     }
-    bigs.erase(bigs.begin() + (long)g);
-    big_pairs.erase(big_pairs.begin() + (long)g);
   }
   std::vector<QItem> items;
   std::vector<QTile> tiles;
@@ -416,19 +459,7 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     }
     items.insert(items.end(), v.begin(), v.end());
   }
-  std::vector<int2> blist;
-  std::vector<long long> booff;
-  std::vector<int> bcount;
-  for (size_t g = 0; g < bigs.size(); g++) {
-    bigs[g].first = (int)blist.size();
-    bigs[g].count = (int)big_pairs[g].size();
-    bcount.push_back(bigs[g].count);
-    for (auto &e : big_pairs[g]) {
-      blist.push_back(e.first);
-      booff.push_back(e.second);
-    }
-  }
-  if (items.size() > (size_t)INT32_MAX || blist.size() > (size_t)INT32_MAX) return fail("too many pairs in one plan");
+  if (items.size() > (size_t)INT32_MAX) return fail("too many pairs in one plan");
   hipSetDevice(q->c.dev);
   // tables for every length in the plan
   for (int lg = 6; lg <= kQMaxLog2; lg++)
@@ -449,7 +480,7 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
       !up(dbcount, bcount.data(), bcount.size() * sizeof(int), "copy four-step counts") ||
       !hip_ok(hipStreamSynchronize(q->c.stream), "hipStreamSynchronize"))
     return -1;
-  q->big = bigs;
+  q->big = lists;
   q->nreq = nreq;
   q->ntiles = (int)tiles.size();
   q->nout = nout;
