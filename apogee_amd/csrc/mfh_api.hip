@@ -258,6 +258,11 @@ void *Ctx::scratch(const char *name, size_t bytes) {
          name, bytes);
     return nullptr;
   }
+  if (capturing) {
+    // an eager call with the same arguments and tuning comes before a capture
+    fail("the context's '%s' buffer (%zu bytes) is not built yet and cannot be while a graph is captured", name, bytes);
+    return nullptr;
+  }
   Buf &b = bufs[name];
   if (b.p) {
     hipStreamSynchronize(stream);
@@ -277,13 +282,20 @@ void *Ctx::scratch(const char *name, size_t bytes) {
   return b.p;
 }
 
+// A kernel, not a memset: callers may record their own launches on a stream in capture.
+__global__ void __launch_bounds__(256) zero_counters_kernel(int *p, size_t n) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
 int *Ctx::part_counters(size_t pairs) {
   const size_t bytes = pairs * sizeof(int);
   const auto found = bufs.find("part_done");
   const bool ready = found != bufs.end() && found->second.p && found->second.bytes >= bytes;
   int *p = (int *)scratch("part_done", bytes);
-  if (p && !ready && !hip_ok(hipMemsetAsync(p, 0, bytes, stream), "hipMemsetAsync")) return nullptr;
-  return p;
+  if (!p || ready) return p;
+  hipLaunchKernelGGL(zero_counters_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, p, pairs);
+  return hip_ok(hipGetLastError(), "zero_counters_kernel") ? p : nullptr;
 }
 
 int Ctx::own_bank(bool templates) {

@@ -605,7 +605,7 @@ int hier_run_cached(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, floa
                                 fbits(coarse_thr), (long long)(intptr_t)out.idx, (long long)(intptr_t)out.val, (long long)(intptr_t)out.rec,
                                 c->coarse_band, dbits(c->coarse_ref_f), c->coarse_prec, fbits(c->coarse_delta),
                                 c->refine_grid_cap, (long long)(intptr_t)c->coarse_tmpl, c->coarse_tpw, c->coarse_rpw, c->coarse_lds,
-                                c->coarse_fuse,
+                                c->coarse_fuse, c->wide, c->big_chunk_bytes,
                                 (long long)(intptr_t)c->data, (long long)(intptr_t)c->tmpl};
   const int par = c->hier_parity;
   if (key == c->graph_key && c->hier_graph[par]) {
