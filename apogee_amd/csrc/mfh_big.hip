@@ -234,26 +234,38 @@ big_cols_kernel(BigArgs a, int np) {
   }
 }
 
-// The last two passes of the one-workgroup transform over row k of its 16 RF
-// rows: 256 points, thread t holding t + 16 u.  Twiddles as there: the third
-// pass's depend on the row only, the fourth's on k + 16 RF t.
+// The table rows of the last two passes of the one-workgroup transform over row
+// k of its 16 RF rows: the third pass's depend on the row only, the fourth's on
+// k + 16 RF t.  Read ahead of the row itself (65536, 160 pairs: rows 19.3 -> 18.7 us).
 template <int RF>
-__device__ __forceinline__ void closing_passes(cf *v, int t, int k, cf *xch, const cf *tw) {
-  using L = TwiddleLayout<4096 * RF>;
-  constexpr int p0 = L::NS0 == 1 ? 1 : 0;  // the table of NS = RF
-  const cf *tw3 = tw + L::offset(p0 + 1), *tw4 = tw + L::offset(p0 + 2);
+struct ClosingTwiddles {
+  cf w3[4], w4[2];  // w^1, w^2, w^4, w^8 and w^1, w^4
+  __device__ __forceinline__ ClosingTwiddles(int t, int k, const cf *tw) {
+    using L = TwiddleLayout<4096 * RF>;
+    constexpr int p0 = L::NS0 == 1 ? 1 : 0;  // the table of NS = RF
+    const cf *tw3 = tw + L::offset(p0 + 1) + k, *tw4 = tw + L::offset(p0 + 2) + k + 16 * RF * t;
+    const cf *e = tw + L::extra() + k;
+    w3[0] = tw3[0];
+    w3[1] = e[0];
+    w3[2] = tw3[16 * RF];
+    w3[3] = e[16 * RF];
+    w4[0] = tw4[0];
+    w4[1] = tw4[256 * RF];
+  }
+};
+
+// Those passes: 256 points, thread t holding t + 16 u.
+template <int RF>
+__device__ __forceinline__ void closing_passes(cf *v, int t, cf *xch, const ClosingTwiddles<RF> &c) {
   cf w[15];
-  const cf *e = tw + L::extra() + k;
-  power_twiddles(w, tw3[k], e[0], tw3[16 * RF + k], e[16 * RF]);
+  power_twiddles(w, c.w3[0], c.w3[1], c.w3[2], c.w3[3]);
 #pragma unroll
   for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
   dft16(v);
   stockham_store<256, 16, 1>(v, t, xch);
-  const int j = k + 16 * RF * t;
-  const cf w1 = tw4[j], w4 = tw4[256 * RF + j];
   __syncthreads();
   stockham_load<256>(v, t, xch);
-  power_twiddles(w, w1, w4);
+  power_twiddles(w, c.w4[0], c.w4[1]);
 #pragma unroll
   for (int r = 1; r < 16; r++) v[r] = cmul(v[r], w[r - 1]);
   dft16(v);
@@ -312,10 +324,18 @@ big_rows_kernel(BigArgs a, BigArgs fin, long long fin_np, int fin_blocks) {
   for (int g = gbeg; g < gend; g++) {
     const int k2 = g * SLOTS + slot;
     cf v[16];
+    auto load = [&]() {
 #pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = Y[(long long)k2 * ROW + t + TPT * u];
-    if constexpr (B::RF > 0) closing_passes<B::RF>(v, t, k2, xch, a.twRow);
-    else inverse_fft<ROW, HOIST>(v, t, xch, a.twRow, wf);
+      for (int u = 0; u < 16; u++) v[u] = Y[(long long)k2 * ROW + t + TPT * u];
+    };
+    if constexpr (B::RF > 0) {
+      const ClosingTwiddles<B::RF> w(t, k2, a.twRow);
+      load();
+      closing_passes<B::RF>(v, t, xch, w);
+    } else {
+      load();
+      inverse_fft<ROW, HOIST>(v, t, xch, a.twRow, wf);
+    }
     // thread t holds z[k2 + ROWS (t + TPT u)]; lags rise with u.  A wave none
     // of whose window lags has |z|^2 above the seed raises no key and records
     // no value, so it skips both steps below (wave-uniform; nonnegative
@@ -440,13 +460,21 @@ __global__ void roots_kernel(cf *out, int L, int period) {
 }
 
 constexpr size_t kLds = 160 * 1024;
-// n = 32768 and 65536, whose calls are small here: a pair's last part merges up to so
-// many table entries (1 x 4 pairs at 65536 32.8 us a call against 34.0 with a finish launch,
-// 2 x 10 at 32768 32.6 against 34.0).  Longer rows keep the finish launch, most
-// of which run inside the next chunk's rows launch: merging there took 2 x 31
-// pairs at 262144 from 104.8 to 102.7, but 1 x 20 from 53.7 to 57.8 and 4 x 64
-// from 321 to 330.
-constexpr size_t kMergeCells = 8192;
+// n = 32768 and 65536: a pair's last part merges the parts' tables where a launch has
+// no more than so many rows workgroups and a pair so many table entries; else a
+// finish launch does.  Each workgroup that counts itself in waits for its
+// entries first, and the next one on its CU for it: with 1024 of them the rows
+// launch takes 14.9 us in place of 9.1, more than the finish launch's 4.6; one
+// workgroup takes 3 us for 4096 entries.  us a call with its wait, merged /
+// finish launch: 65536, 64 bins, threshold 5.5: 4 pairs (64 workgroups) 23.3 /
+// 24.3, 8 24.9 / 24.9, 16 29.1 / 27.6; without a threshold 64 pairs 45.6 / 43.5;
+// 4 pairs of 256 bins 31.6 / 28.5; 32768, one bin: 8 pairs 21.8 / 22.5, 16 23.8
+// / 23.6, 64 33.0 / 32.1; several calls on their way gain another 0.7.  Longer
+// rows keep the finish launch, most of which run inside the next chunk's rows
+// launch: merging there took 2 x 31 pairs at 262144 from 104.8 to 102.7, but
+// 1 x 20 from 53.7 to 57.8 and 4 x 64 from 321 to 330.
+constexpr long long kMergeBlocks = 128;
+constexpr size_t kMergeCells = 1024;
 // Walking pairs pays from a good third more tiles than a launch has resident (us a
 // call, walk / one tile each; tiles): 1280 49.5 / 48.2 and 53.9 / 53.7, 1440 57.6 /
 // 60.2, 1536 66.7 / 67.5, 1792 67.7 / 69.0, 3968 104.8 / 111.
@@ -521,7 +549,7 @@ int big_buffers(Ctx *c, long long total, size_t nb_total, BigArgs &a, BigBuffers
   if (B::RF && nsplit > 1) {
     a.done = c->part_counters((size_t)b.chunk);  // in any case: a later, captured call may have fewer bins
     if (!a.done) return -1;
-    if (nb_piece * nsplit > kMergeCells) a.done = nullptr;
+    if (b.chunk * nsplit > kMergeBlocks || nb_piece * nsplit > kMergeCells) a.done = nullptr;
   }
   return 0;
 }
