@@ -649,7 +649,7 @@ extern "C" int mfh_set_tuning(mfh_ctx *ctx, const char *key, long value) {
     return 0;
   }
   if (!strcmp(key, "wide")) {
-    if (value < 0 || value > 2) return fail("wide must be 0 (by the pair count), 1 (always) or 2 (never)");
+    if (value < 0 || value > 2) return fail("wide must be 0 (by pairs, bins and threshold), 1 (always) or 2 (never)");
     c->wide = (int)value;
     return 0;
   }

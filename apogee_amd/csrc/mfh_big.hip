@@ -663,11 +663,11 @@ static int reserve_shape(Ctx *c, long long pairs, size_t nb) {
   return big_buffers<B>(c, pairs, nb, a, b);
 }
 
-int big_reserve(Ctx *c, size_t n, const FlatRun &r, long long pairs) {
+int big_reserve(Ctx *c, size_t n, const FlatRun &r) {
   const size_t nb = (r.we - r.ws + r.binsize - 1) / r.binsize;
   switch (n) {
-    case 32768: return reserve_shape<BigShape<0, 8>>(c, pairs, nb);
-    case 65536: return reserve_shape<BigShape<0, 16>>(c, pairs, nb);
+    case 32768: return reserve_shape<BigShape<0, 8>>(c, r.list_cap, nb);
+    case 65536: return reserve_shape<BigShape<0, 16>>(c, r.list_cap, nb);
     default: return 0;
   }
 }

@@ -260,14 +260,13 @@ int launch_flat(Ctx *c, size_t n, const FlatRun &r) {
   // allocation-free call over part of the bank the one that this call does
   // not: both find their buffers after one call over the whole.
   if (r.list && r.hint && !c->capturing && !c->no_alloc) {
-    const long long few = std::min<long long>(r.list_cap, wide_min_pairs(n) - 1);
-    if (wide_reserve(c, n, q) < 0 || (few > 0 && big_reserve(c, n, q, few) < 0)) return -1;
+    if (wide_reserve(c, n, q) < 0 || (two_paths(n) && big_reserve(c, n, q) < 0)) return -1;
   }
   bool wide = wide_takes(c, n, q);
   // ... and with more bins than that call had, whichever of the two holds them
   // (their results are the same bits)
   if (r.list && c->no_alloc && two_paths(n) &&
-      (wide ? wide_reserve(c, n, q) : big_reserve(c, n, q, r.list_cap)) < 0)
+      (wide ? wide_reserve(c, n, q) : big_reserve(c, n, q)) < 0)
     wide = !wide;
   if (wide) return launch_wide(c, n, q);
   switch (n) {

@@ -63,7 +63,7 @@ struct Ctx {
   // two-kernel lengths (n >= 32768): roots built, scratch budget per chunk
   bool big_roots_ready[16] = {};  // by log2 of the column length
   long long big_chunk_bytes = 128ll << 20;  // measured best on gfx950 (256: +7%, 64: +16%)
-  int wide = 0;  // n = 8192 ... 65536 through launch_wide: 0 by the pair count, 1 always, 2 never
+  int wide = 0;  // n = 8192 ... 65536 through launch_wide: 0 by pairs, bins and threshold (wide_takes), 1 always, 2 never
   int refine_grid_cap = 2048;  // workgroups of a list-driven (refine) launch, at most
   // pinned host word holding the last hierarchical refine's survivor count,
   // written by that launch (a sizing hint only: results never depend on it)
@@ -222,15 +222,14 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
 // captured or allocation-free call of a list that may take either path).
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r);
 size_t wide_table_bins(size_t n);    // bins of one launch
-long long wide_min_pairs(size_t n);  // pairs from which an automatic run takes it (0: no such length)
 int launch_wide(Ctx *c, size_t n, const FlatRun &r);
 int wide_reserve(Ctx *c, size_t n, const FlatRun &r);
 // The two-kernel flat filter for n >= 32768.
 int launch_big(Ctx *c, size_t n, const FlatRun &r);
-// Its buffers for up to `pairs` pairs of r made in advance (n = 32768 and 65536, where
-// an allocation-free call may take either path).  With Ctx::no_alloc set: < 0 if
+// Its buffers for a list run made in advance (n = 32768 and 65536, where an
+// allocation-free call may take either path).  With Ctx::no_alloc set: < 0 if
 // they are not there.
-int big_reserve(Ctx *c, size_t n, const FlatRun &r, long long pairs);
+int big_reserve(Ctx *c, size_t n, const FlatRun &r);
 // Four-step root tables for n = n1 * 256: w_n1^h (h < n1) then w_n^l (l < 256),
 // FP64-generated once per context.
 const cf *big_roots(Ctx *c, int n1);

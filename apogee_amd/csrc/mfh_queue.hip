@@ -70,6 +70,9 @@ struct QTile {
 
 constexpr int kQThreads = 1024;
 constexpr int kQMaxLog2 = 14;  // longest length of the persistent kernel
+// pairs of a group of 8192 or 16384 points from which a list launch pays (the
+// one-workgroup path takes lists of so many)
+constexpr long long kQListPairs = 257;
 // exchange space of a tile: 1024 lanes x 16 points, padded by 1/16, plus one
 // element per slot where slots share a wave (largest at n = 64: 256 slots)
 template <int N>
@@ -415,7 +418,7 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
   std::vector<int> bcount;
   std::vector<Queue::BigGroup> lists;
   for (auto &G : bigs) {
-    G.list = ilog2(G.n) > kQMaxLog2 || G.pairs >= wide_min_pairs((size_t)G.n);
+    G.list = ilog2(G.n) > kQMaxLog2 || G.pairs >= kQListPairs;
     if (!G.list) continue;
     if (listed + G.pairs > INT32_MAX) return fail("too many pairs in one plan");
     G.first = (int)listed;

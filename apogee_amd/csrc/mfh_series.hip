@@ -266,6 +266,9 @@ long run_series(Ctx *c, bool hier, const void *series_c64, size_t nseries, int s
     same = same && win_start[b] == win_start[0] && win_end[b] == win_end[0];
     aligned = aligned && win_start[b] % 64 == 0 && std::min(win_end[b], n) % 64 == 0;
   }
+  // as the launch below asks for its path
+  base.ws = win_start[0];
+  base.we = std::min(win_end[0], n);
   uint2 *win = nullptr;
   if (!hier && !same && nblocks <= mfh::BlockStarts::kInline && nb <= mfh::flat_row_window_bins(c, n, base)) {
     win = (uint2 *)c->scratch("series_win", mfh::BlockStarts::kInline * sizeof(uint2));

@@ -44,13 +44,40 @@ namespace mfh {
 
 namespace {
 
-// From how many pairs a call takes this path, by length 8192 ... 65536.  Below,
-// more threads per pair win: at 8192 and 16384 one workgroup per CU of the
-// 16-point kernel (256 pairs: 8.2 against 9.4 us and 12.1 against 12.4; 384
-// pairs: 11.5 against 10.8 and 22.1 against 17.6), at 32768 and 65536 the
-// two-kernel path (24 pairs: 14.3 against 14.8 us, 32: 16.0 against 15.0;
-// 32 pairs: 24.6 against 24.4, 48: 28.0 against 24.4).
-constexpr long long kWideMinPairs[4] = {257, 257, 28, 32};
+// From how many pairs a call takes this path at 8192, 16384 and 32768.  Below, more
+// threads per pair win: at 8192 and 16384 one workgroup per CU of the 16-point
+// kernel (256 pairs: 8.2 against 9.4 us and 12.1 against 12.4; 384 pairs: 11.5
+// against 10.8 and 22.1 against 17.6), at 32768 the two-kernel path (24 pairs:
+// 16.8 against 15.8 us, but 25.7 against 26.3 with three filters in turn; 32:
+// 20.6 and 17.3, 28.5 and 27.2).
+// The second column: without a threshold and with several bins.  Every sample is
+// a candidate then, which costs a thread with 32 of them more (8192, aligned
+// bins, which the 16-point kernel selects in runs: 512 pairs 14.4 against 16.8 us,
+// 600 22.2 and 19.4; 32768: 40 pairs 23.9 and 25.1, 88 in turn 38.6 and 38.2,
+// 104 41.4 and 38.4).
+constexpr long long kWideMinPairs[3][2] = {{257, 513}, {257, 257}, {32, 104}};
+
+// n = 65536: one workgroup of 1024 threads fills a CU, so pairs run in rounds of
+// 128, each 25 us (36 with every sample a candidate), while the two-kernel
+// path takes 0.17 (0.22) us a pair and 8 more per 256, one chunk of its
+// scratch.  A round that the call does not fill must therefore hold enough
+// pairs.  us a call, this path / two kernels, in brackets with three filters in
+// turn, whose scratch leaves the caches; threshold 5.5, 64 bins: 64 pairs 26.9 /
+// 30.8 (39.4 / 37.0), 72 26.2 / 32.2 (39.3 / 39.6); 132 51.1 / 41.6 (61.6 / 56.9),
+// 160 50.2 / 45.8 (62.0 / 70.2), 192 51.0 / 49.3 (62.1 / 79.0); 260 74.8 / 71.7,
+// 268 74.4 / 72.6 (86.0 / 112.2); 388 98.1 / 97.3; 512 101 / 119 (113 / 182).
+// Without a threshold: 64 pairs 37.2 / 34.5 (50.9 / 40.2), 104 40.2 / 42.4 (51.3 /
+// 51.7); 256 76.2 / 75.6 (87.6 / 112); 352 110.5 / 107.2 (122 / 155), 368 111.4 /
+// 110.1; 512 148 / 142 (160 / 207); from eight rounds on, where the spectra
+// leave the caches, 1000 pairs 288 / 329.
+bool wide_rounds_pay(long long pairs, bool dense) {
+  constexpr long long kRound = 128;
+  const long long rounds = (pairs + kRound - 1) / kRound, last = pairs - (rounds - 1) * kRound;
+  // after an odd number the other path has a chunk that is partly filled
+  if (dense) return rounds >= 8 || (rounds % 2 == 1 && last >= 104);
+  constexpr int kFill[3] = {72, 64, 12};
+  return rounds > 3 || (rounds > 0 && last >= kFill[rounds - 1]);
+}
 
 struct WideArgs {
   FlatArgs f;              // rows, window, bins, outputs, list
@@ -746,8 +773,6 @@ size_t wide_table_bins(size_t n) {
   }
 }
 
-long long wide_min_pairs(size_t n) { return n < 8192 || n > 65536 ? 0 : kWideMinPairs[ilog2((int)n) - 13]; }
-
 bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   if (n < 8192 || n > 65536 || c->wide == 2) return false;
   if (c->wide == 1) return true;
@@ -757,7 +782,11 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   // it takes, so it goes by the list's capacity
   if (r.list && r.hint && !c->capturing && !c->no_alloc)
     pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
-  return pairs >= wide_min_pairs(n);
+  bool dense = !(r.threshold > 0.f) && r.we - r.ws > r.binsize;
+  if (n == 65536) return wide_rounds_pay(pairs, dense);
+  // a list's 16-point launches select without runs; bins off the 64-lag grid too
+  if (n == 8192) dense = dense && !r.list && r.binsize % 64 == 0 && r.ws % 64 == 0 && r.we % 64 == 0;
+  return pairs >= kWideMinPairs[ilog2((int)n) - 13][dense];
 }
 
 int launch_wide(Ctx *c, size_t n, const FlatRun &r) {

@@ -348,7 +348,7 @@ long mfh_hier_run_series_rec(mfh_ctx *ctx, const void *series_c64, size_t nserie
  * survivors in the same launch; with the FP32 screen, gate and refine share a
  * launch, which at bands up to 256 also screens), "big_chunk_mb" (scratch
  * per column / row launch pair of the two-kernel path), "wide" (n = 8192 ... 65536, one
- * workgroup per pair or half of one: 0 = by the pair count, 1 = always,
+ * workgroup per pair or half of one: 0 = by pairs, bins and threshold, 1 = always,
  * 2 = never; results are the same), "totals" (1 by default; 0: runs with host
  * results return 0 instead of the number of reported bins unless per-pair
  * counts are asked for, which saves a pass over the results), "graphs" (0/1: replay the
