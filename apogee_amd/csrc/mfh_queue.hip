@@ -15,8 +15,8 @@
 // the flat filter's own launches for those lengths, queued just before the
 // persistent launch in the same stream and graph: n >= 32768 always, 8192 and
 // 16384 where a group of equal (n, binsize, threshold, window) has enough pairs
-// for the one-workgroup path (its 32 points per thread and two workgroups per
-// CU against one 1024-lane workgroup here).
+// (list_pays) for the one-workgroup path (its 32 points per thread and two
+// workgroups per CU against one 1024-lane workgroup here).
 //
 // Arithmetic.  Every pair runs the same product, transforms, twiddle tables
 // and exact key rule as the per-request flat filter, so indices and values
@@ -70,9 +70,6 @@ struct QTile {
 
 constexpr int kQThreads = 1024;
 constexpr int kQMaxLog2 = 14;  // longest length of the persistent kernel
-// pairs of a group of 8192 or 16384 points from which a list launch pays (the
-// one-workgroup path takes lists of so many)
-constexpr long long kQListPairs = 257;
 // exchange space of a tile: 1024 lanes x 16 points, padded by 1/16, plus one
 // element per slot where slots share a wave (largest at n = 64: 256 slots)
 template <int N>
@@ -270,6 +267,25 @@ struct Queue {
   long prof_runs = 0;  // runs recorded while event timing is on
 };
 
+// Whether a group of 8192 or 16384 points gets a list launch of its own.  Its
+// pairs would otherwise fill workgroups that the persistent launch keeps busy
+// anyway, while list launches run one after another, each with a last wave of
+// workgroups that is partly empty.  Against the persistent launch, one to ten
+// such groups, alone or with 500 or 2000 shorter requests beside them:
+//   threshold 5.5: 8192, 257 pairs 1.11 of its time at worst, 350 1.02, 450
+//   0.94; 16384, 257 1.03, 300 0.99, 400 0.94 (at best 0.6 throughout);
+//   without a threshold: 8192, 350 1.06, 512 0.94; 16384, 300 1.11, 400 0.95.
+// Eight bins over the whole row, which the persistent launch selects in runs:
+//   threshold 5.5: 8192, 400 1.11, 512 0.98; 16384, 300 1.17, 400 1.01;
+//   without one: 8192, 257 1.9, 600 1.18, 1024 0.96; 16384, 257 1.6, 600 1.2, 1024 0.94.
+bool list_pays(const Queue::BigGroup &G) {
+  if (ilog2(G.n) > kQMaxLog2) return true;
+  const bool runs = G.ws == 0 && G.we == G.n && G.binsize * 8 == G.n, dense = !(G.threshold > 0.f);
+  if (runs && dense) return G.pairs >= 1024;
+  if (runs || dense) return G.pairs >= (G.n == 8192 ? 512 : 400);
+  return G.pairs >= (G.n == 8192 ? 350 : 300);
+}
+
 // Finds a request's group among those seen so far, in constant time: requests
 // with a window or threshold of their own are a group each (40000 of them plan
 // in 2 ms; a walk over the groups took 1.2 s).
@@ -412,13 +428,12 @@ extern "C" long long mfh_queue_plan(mfh_queue *queue, int nreq, const int64_t *n
     nout += (long long)ncand[r] * nb;
     npairs += ncand[r];
   }
-  // the groups that get a list launch: not those of 8192 and 16384 too small for
-  // the one-workgroup path
+  // the groups that get a list launch
   long long listed = 0;
   std::vector<int> bcount;
   std::vector<Queue::BigGroup> lists;
   for (auto &G : bigs) {
-    G.list = ilog2(G.n) > kQMaxLog2 || G.pairs >= kQListPairs;
+    G.list = list_pays(G);
     if (!G.list) continue;
     if (listed + G.pairs > INT32_MAX) return fail("too many pairs in one plan");
     G.first = (int)listed;
