@@ -260,7 +260,12 @@ int launch_flat(Ctx *c, size_t n, const FlatRun &r) {
   // allocation-free call over part of the bank the one that this call does
   // not: both find their buffers after one call over the whole.
   if (r.list && r.hint && !c->capturing && !c->no_alloc) {
-    if (wide_reserve(c, n, q) < 0 || (two_paths(n) && big_reserve(c, n, q) < 0)) return -1;
+    const size_t nb = (we - r.ws + r.binsize - 1) / r.binsize;
+    Ctx::ListReady &ready = c->list_ready;
+    if (r.list_cap != ready.pairs || nb != ready.bins || c->big_chunk_bytes != ready.chunk_bytes) {
+      if (wide_reserve(c, n, q) < 0 || (two_paths(n) && big_reserve(c, n, q) < 0)) return -1;
+      ready = {r.list_cap, nb, c->big_chunk_bytes};
+    }
   }
   bool wide = wide_takes(c, n, q);
   // ... and with more bins than that call had, whichever of the two holds them

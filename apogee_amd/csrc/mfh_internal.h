@@ -94,6 +94,12 @@ struct Ctx {
   std::map<std::string, Buf> bufs;
   // Device buffer `name`, grown on demand (contents not preserved on growth).
   void *scratch(const char *name, size_t bytes);
+  // the list run that launch_flat reserved buffers for last (buffers only grow)
+  struct ListReady {
+    long long pairs = 0;
+    size_t bins = 0;
+    long long chunk_bytes = 0;
+  } list_ready;
   // one counter per pair of a launch for part_is_last, 0 between launches
   int *part_counters(size_t pairs);
 

@@ -685,7 +685,7 @@ WideKernel wide_pick(Ctx *c, size_t nb, bool dense) {
 template <class W, bool LIST>
 int wide_tables(Ctx *c, WideArgs &wa, long long total, size_t nb, long long &chunk) {
   chunk = std::max<long long>(1, std::min<long long>(total, (64ll << 20) / ((long long)W::S * (long long)nb * 16)));
-  if (c->no_alloc) {  // the tables that are there, in more launches if need be
+  if (c->no_alloc || c->capturing) {  // the tables that are there, in more launches if need be
     const auto have = c->bufs.find("wide_key");
     const long long fit = have == c->bufs.end() ? 0 : (long long)(have->second.bytes / (W::S * nb * sizeof(uint64_t)));
     if (fit > 0) chunk = std::min(chunk, fit);
@@ -780,9 +780,15 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   // a list's length as of the previous call (results never depend on it); a
   // captured or allocation-free call must find the buffers of the route that
   // it takes, so it goes by the list's capacity
-  if (r.list && r.hint && !c->capturing && !c->no_alloc)
-    pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
   bool dense = !(r.threshold > 0.f) && r.we - r.ws > r.binsize;
+  if (r.list && r.hint && !c->capturing && !c->no_alloc) {
+    pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
+    // the two-kernel path launches every chunk that the list could fill: 65536, 640
+    // pairs of which 0 / 24 / 136 are left, one bin: 37 / 43 / 63 us a
+    // hierarchical call, here 21 / 38 / 62
+    if (n >= 32768 && !dense && (long long)r.list_cap * (long long)n * (long long)sizeof(cf) > c->big_chunk_bytes)
+      return true;
+  }
   if (n == 65536) return wide_rounds_pay(pairs, dense);
   // a list's 16-point launches select without runs; bins off the 64-lag grid too
   if (n == 8192) dense = dense && !r.list && r.binsize % 64 == 0 && r.ws % 64 == 0 && r.we % 64 == 0;
