@@ -70,9 +70,7 @@ int flat_base_args(Ctx *c, size_t n, const FlatRun &r, size_t ws, size_t we, siz
   a.list_ooff = r.list_ooff;
   a.zero = bin0 == 0 ? r.zero : nullptr;
   a.hint = bin0 == 0 ? r.hint : nullptr;
-  int dpw = c->tune_dpw;
-  if (dpw <= 0) dpw = std::min(r.nd, 4);
-  a.dpw = dpw;
+  a.dpw = 1;
   return 0;
 }
 
@@ -98,13 +96,13 @@ int launch_n(Ctx *c, const FlatRun &r, size_t ws, size_t we, size_t nb_total, si
     }
     grid = dim3((unsigned)std::max(1, std::min(want, c->refine_grid_cap)), 1);
   } else {
-    if ((r.nd + a.dpw - 1) / a.dpw > 65535) return fail("too many data rows per launch (%d)", r.nd);
     // A tile of several rows saves nothing but workgroups (the template is
     // read again for each row, from the caches): one row per workgroup unless
     // tuned otherwise (n = 4096, eight bins, calls with device results: 64 x 32
     // pairs 46.7 us with tiles of four, which leave half of the chip idle,
-    // and 40.5 with one; 16 x 16 43.4 and 28.0; 64 x 512 256.6 and 246.5), and
-    // a tuned tile only while it leaves 1024 workgroups
+    // and 40.5 with one; 16 x 16 43.4 and 28.0; 64 x 512 256.6 and 246.5), a
+    // tuned tile only while it leaves 1024 workgroups, and as many rows as it
+    // takes to keep the grid's second dimension within 65535
     const unsigned groups = (unsigned)((r.nt + S::SLOTS - 1) / S::SLOTS);
     int dpw = c->tune_dpw > 0 ? c->tune_dpw : 1;
     while (dpw > 1 && (long long)groups * ((r.nd + dpw - 1) / dpw) < 1024) dpw /= 2;

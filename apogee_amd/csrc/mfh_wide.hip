@@ -742,9 +742,6 @@ int wide_run(Ctx *c, const FlatRun &r) {
     const size_t ws = r.ws + b0 * r.binsize;
     const size_t we = std::min(r.we, ws + cnt * r.binsize);
     if (flat_base_args(c, W::N, r, ws, we, nb_total, b0, cnt, wa.f) < 0) return -1;
-    // the limit of the 16-point kernel, whichever of the two runs
-    if (!r.list && W::S == 1 && (r.nd + wa.f.dpw - 1) / wa.f.dpw > 65535)
-      return fail("too many data rows per launch (%d)", r.nd);
     if ((r.list ? wide_piece<W, true>(c, wa, total, cnt) : wide_piece<W, false>(c, wa, total, cnt)) < 0) return -1;
   }
   return 0;
