@@ -123,6 +123,15 @@ def _median_ms(fn, reps, ctx, name):
     return statistics.median(times)
 
 
+def flat_tiles(n, nd, nt):
+    """The ``dpw`` candidates that launch different tiles at this shape: the
+    filter halves a tile that leaves fewer than 1024 workgroups, and from
+    n = 8192 on calls large enough for one take a path without tiles."""
+    groups = -(-nt // max(1, 4096 // n))
+    keep = [d for d in CANDIDATES["flat"]["dpw"] if d == 1 or (d <= nd and groups * -(-nd // d) >= 1024)]
+    return keep if n < 8192 else [1]
+
+
 def _tune_flat(device, n, nd, nt, binsize, reps, rng):
     import numpy as np
     from . import _hip
@@ -134,9 +143,7 @@ def _tune_flat(device, n, nd, nt, binsize, reps, rng):
     idx = torch.empty(nd * nt * nb, dtype=torch.int64, device="cuda:%d" % device)
     val = torch.empty(nd * nt * nb, dtype=torch.complex64, device="cuda:%d" % device)
     ms = {}
-    for dpw in CANDIDATES["flat"]["dpw"]:
-        if dpw > nd:
-            continue
+    for dpw in flat_tiles(n, nd, nt):
         ctx.set_tuning("dpw", dpw)
         run = lambda: ctx.peaks_async(0, nd, 0, nt, binsize, 0.0, 0, n, idx.data_ptr(), val.data_ptr())
         run()
@@ -152,6 +159,8 @@ def _tune_big(device, n, nd, nt, binsize, reps, rng):
     import numpy as np
     from . import _hip
     ctx = _hip.Context(device, n, nd, nt)
+    if n <= 65536:
+        ctx.set_tuning("wide", 2)  # the two-kernel path, whichever these shapes take
     ctx.set_rows("data", 0, (rng.standard_normal((nd, n)) + 1j * rng.standard_normal((nd, n))).astype(np.complex64))
     ctx.set_rows("template", 0, (rng.standard_normal((nt, n)) + 1j * rng.standard_normal((nt, n))).astype(np.complex64))
     import torch
