@@ -278,10 +278,11 @@ struct Queue {
 // Eight bins over the whole row, which the persistent launch selects in runs:
 //   threshold 5.5: 8192, 400 1.11, 512 0.98; 16384, 300 1.17, 400 1.01;
 //   without one: 8192, 257 1.9, 600 1.18, 1024 0.96; 16384, 257 1.6, 600 1.2, 1024 0.94.
+// Many small bins without a threshold: 8192, 24 lags, 512 1.08; 16384, 400 1.16.
 bool list_pays(const Queue::BigGroup &G) {
   if (ilog2(G.n) > kQMaxLog2) return true;
   const bool runs = G.ws == 0 && G.we == G.n && G.binsize * 8 == G.n, dense = !(G.threshold > 0.f);
-  if (runs && dense) return G.pairs >= 1024;
+  if (dense && (runs || (G.binsize <= 128 && G.we - G.ws > G.binsize))) return G.pairs >= 1024;
   if (runs || dense) return G.pairs >= (G.n == 8192 ? 512 : 400);
   return G.pairs >= (G.n == 8192 ? 350 : 300);
 }

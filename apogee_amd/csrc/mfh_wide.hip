@@ -50,12 +50,7 @@ namespace {
 // against 10.8 and 22.1 against 17.6), at 32768 the two-kernel path (24 pairs:
 // 16.8 against 15.8 us, but 25.7 against 26.3 with three filters in turn; 32:
 // 20.6 and 17.3, 28.5 and 27.2).
-// The second column: without a threshold and with several bins.  Every sample is
-// a candidate then, which costs a thread with 32 of them more (8192, aligned
-// bins, which the 16-point kernel selects in runs: 512 pairs 14.4 against 16.8 us,
-// 600 22.2 and 19.4; 32768: 40 pairs 23.9 and 25.1, 88 in turn 38.6 and 38.2,
-// 104 41.4 and 38.4).
-constexpr long long kWideMinPairs[3][2] = {{257, 513}, {257, 257}, {32, 104}};
+constexpr long long kWideMinPairs[3] = {257, 257, 32};
 
 // n = 65536: one workgroup of 1024 threads fills a CU, so pairs run in rounds of
 // 128, each 25 us (36 with every sample a candidate), while the two-kernel
@@ -67,14 +62,13 @@ constexpr long long kWideMinPairs[3][2] = {{257, 513}, {257, 257}, {32, 104}};
 // 160 50.2 / 45.8 (62.0 / 70.2), 192 51.0 / 49.3 (62.1 / 79.0); 260 74.8 / 71.7,
 // 268 74.4 / 72.6 (86.0 / 112.2); 388 98.1 / 97.3; 512 101 / 119 (113 / 182).
 // Without a threshold: 64 pairs 37.2 / 34.5 (50.9 / 40.2), 104 40.2 / 42.4 (51.3 /
-// 51.7); 256 76.2 / 75.6 (87.6 / 112); 352 110.5 / 107.2 (122 / 155), 368 111.4 /
-// 110.1; 512 148 / 142 (160 / 207); from eight rounds on, where the spectra
-// leave the caches, 1000 pairs 288 / 329.
+// 51.7); 256 76.2 / 75.6 (87.6 / 112); 352 110.5 / 107.2 (122 / 155); 512 148 /
+// 142 (160 / 207); from eight rounds on, where the spectra leave the caches,
+// 1000 pairs 288 / 329.
 bool wide_rounds_pay(long long pairs, bool dense) {
   constexpr long long kRound = 128;
   const long long rounds = (pairs + kRound - 1) / kRound, last = pairs - (rounds - 1) * kRound;
-  // after an odd number the other path has a chunk that is partly filled
-  if (dense) return rounds >= 8 || (rounds % 2 == 1 && last >= 104);
+  if (dense) return rounds >= 8 || (rounds == 1 && last >= 104);
   constexpr int kFill[3] = {72, 64, 12};
   return rounds > 3 || (rounds > 0 && last >= kFill[rounds - 1]);
 }
@@ -496,10 +490,13 @@ __device__ __forceinline__ void wide_select(const FlatArgs &a, const cf *v, uint
 }
 
 // Write the peaks of the bins whose winning lag this wave holds, at o + bin of
-// the outputs (S = 1) or only their values, to pval (the keys go apart).  Up to kWideLook bins, each lane looks at one
-// bin's key and the wave then visits its own winners; past that the samples
-// are fewer than the bins, and the `hot` ones look up theirs.
-constexpr int kWideLook = 2048;
+// the outputs (S = 1) or only their values, to pval (the keys go apart).  Up to
+// kWideLook bins, each lane looks at one bin's key and the wave then visits its
+// own winners one by one; past that the `hot` samples, 32 at most, look up
+// theirs.  The line: without a threshold a wave of n = 8192 wins a quarter of the
+// bins (2048 bins, 2052 pairs: 2.5 times the 16-point kernel's time by visits,
+// 0.74 by lookups; 256 bins 1.05 and 1.05; 128 bins 0.88 and 0.94).
+constexpr int kWideLook = 256;
 template <class W, bool ONE>
 __device__ __forceinline__ void wide_write(const FlatArgs &a, const WideSamples &v, uint32_t hot, int t, int h,
                                            int lane, int nb, const uint64_t *bins, long long o, cf *pval) {
@@ -777,7 +774,9 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   // a list's length as of the previous call (results never depend on it); a
   // captured or allocation-free call must find the buffers of the route that
   // it takes, so it goes by the list's capacity
-  bool dense = !(r.threshold > 0.f) && r.we - r.ws > r.binsize;
+  // without a threshold and with several bins every sample is a candidate, which
+  // costs a thread with 32 of them more
+  const bool multi = r.we - r.ws > r.binsize, dense = multi && !(r.threshold > 0.f);
   if (r.list && r.hint && !c->capturing && !c->no_alloc) {
     pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
     // the two-kernel path launches every chunk that the list could fill: 65536, 640
@@ -786,10 +785,33 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
     if (n >= 32768 && !dense && (long long)r.list_cap * (long long)n * (long long)sizeof(cf) > c->big_chunk_bytes)
       return true;
   }
-  if (n == 65536) return wide_rounds_pay(pairs, dense);
-  // a list's 16-point launches select without runs; bins off the 64-lag grid too
-  if (n == 8192) dense = dense && !r.list && r.binsize % 64 == 0 && r.ws % 64 == 0 && r.we % 64 == 0;
-  return pairs >= kWideMinPairs[ilog2((int)n) - 13][dense];
+  // n = 8192, several bins: the 16-point kernel selects bins on the 64-lag grid in
+  // runs, and holds its own to two workgroups per CU (us, here / there: without a
+  // threshold, 1024-lag bins, 512 pairs 16.8 / 14.4, 600 19.4 / 22.2; threshold 3,
+  // 1% of the samples, 400 pairs 1.16 of its time, 520 1.01).  Bins that several
+  // lanes of a wave share but a wave straddles: 24 lags, 1030 pairs 1.19.
+  if (n == 8192 && multi && !r.list) {
+    const bool runs = r.binsize % 64 == 0 && r.ws % 64 == 0 && r.we % 64 == 0;
+    if (dense && r.binsize > 8 && r.binsize < 64) return false;
+    return pairs >= (dense && !runs && r.binsize >= 200 ? kWideMinPairs[0] : 513);
+  }
+  if (n <= 16384 || !multi) return n == 65536 ? wide_rounds_pay(pairs, false) : pairs >= kWideMinPairs[ilog2((int)n) - 13];
+  // n = 32768 and 65536, several bins.  Tables that fill most of the LDS leave the
+  // rows of two kernels few workgroups per CU: 65536, without a threshold, 16
+  // lags to a bin, 64 pairs 0.83 of their time, 132 0.91; 8 lags, 24 pairs 0.93;
+  // 32768, 8 lags, 40 pairs 0.99.
+  const size_t nb = (r.we - r.ws + r.binsize - 1) / r.binsize;
+  if (n == 65536 && nb > 3000) return pairs >= (nb >= 8192 ? 24 : 64);
+  if (n == 32768 && nb >= 4096) return pairs >= (dense ? 48 : 40);
+  // A wave's lags at one step span 128: without a threshold, bins down to a few
+  // lanes wide straddle it (64 lags: 32768, 130 pairs 1.37 of the other path's
+  // time, 600 1.17, 1030 0.91; 65536, 128 pairs 1.16, 1000 1.11, 2000 1.22; 300
+  // lags: 32768, 260 pairs 1.10; 65536, 104 1.06, 1000 0.85; 512: 0.80 ... 1.0).
+  if (n == 32768) return pairs >= (!dense ? 56 : r.binsize > 16 && r.binsize <= 400 ? 1024 : 104);
+  if (dense && r.binsize <= (pairs >= 1024 ? 200 : 400)) return false;
+  // with a threshold that 1% of the samples beat, a round costs up to 1.2 times
+  // what the lines are for; search thresholds leave 1e-4 and fewer
+  return wide_rounds_pay(pairs, dense);
 }
 
 int launch_wide(Ctx *c, size_t n, const FlatRun &r) {

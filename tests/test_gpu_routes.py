@@ -61,3 +61,31 @@ def test_series_windows_on_either_path(n, nt, gpu_device):
         for b in range(4):
             one = c.run_series(x, starts[b:b + 1], lo[b:b + 1], hi[b:b + 1], 0, nt, bs, thr, records=mf.PEAK_DTYPE)[0]
             assert np.array_equal(got[0][b:b + 1], one), (n, bs, thr, b)
+
+
+@pytest.mark.parametrize("n", [8192, 16384, 32768, 65536])
+def test_winners_found_either_way(n, gpu_device):
+    """256 bins, whose winners a wave visits, and a few more, which the samples
+    look up: all samples candidates, some, a few."""
+    D, T = bank(n, 2, 3, n + 8)
+    f = mf.MatchedFilter(n, 2, 3)
+    f.set_data(D)
+    f.set_templates(T)
+    for bs, window in [(n // 256, None), (n // 256 - 1, None), (n // 256, (1, n)), (17, (3, 3 + 17 * 256 + 1))]:
+        for thr in (0.0, 2.5, 5.0):
+            wide, two = both(f, binsize=bs, threshold=thr, window=window)
+            assert np.array_equal(wide, two), (n, bs, window, thr)
+
+
+@pytest.mark.parametrize("n,pairs,bs", [(8192, 600, 24), (8192, 300, 200), (32768, 48, 8), (32768, 130, 100), (65536, 66, 16),
+                                        (65536, 120, 128)])
+def test_automatic_choice_by_bin_width(n, pairs, bs, gpu_device):
+    D, T = bank(n, 1, pairs, n + 7)
+    f = mf.MatchedFilter(n, 1, pairs)
+    f.set_data(D)
+    f.set_templates(T)
+    for thr in (0.0, 4.0):
+        f._gpu.set_tuning("wide", 0)
+        auto = f.run(binsize=bs, threshold=thr)
+        wide, two = both(f, binsize=bs, threshold=thr)
+        assert np.array_equal(auto, wide) and np.array_equal(auto, two), thr
