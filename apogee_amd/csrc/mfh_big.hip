@@ -8,16 +8,16 @@
 // of the one-workgroup transform (mfh_wide.hip), the first two in kernel A
 // (256 columns of 16 RF points), the last two in kernel B (16 RF rows of 256
 // points), with the same arithmetic and so the same bits.  Spread over many
-// workgroups, one pair takes 14 us instead of 33 at n = 65536; from about 30 pairs
-// on the scratch round trip costs more than it gives.
-// Kernel A forms the product D*conj(T) on load, runs 256-point inverse FFTs
-// over 16 columns per workgroup and writes Y k2-major to scratch (each
-// 16-lane group writes 128 contiguous bytes).  Kernel B gives each pair a few
-// workgroups that walk k2 in groups, run the row transforms, and keep
-// a per-bin (key, value) table in LDS: keys rise by ds_max_u64, and after
-// each group the lane holding the bin's key writes its value, so the table
-// always pairs the largest |z|^2 (lowest lag among equals) with its own z.
-// Only the final per-bin result leaves the chip.
+// workgroups, one pair takes 14 us instead of 33 at n = 65536; from some 30 (70 at
+// 65536) pairs on the scratch round trip costs more than it gives (wide_takes).
+// Kernel A forms the product D*conj(T) on load, runs the column transforms (256
+// points, 16 RF at 32768 and 65536) over 16 columns per workgroup and writes Y
+// k2-major to scratch (each 16-lane group writes 128 contiguous bytes).
+// Kernel B gives each pair a few workgroups that walk k2 in groups, run the row
+// transforms, and keep a per-bin (key, value) table in LDS: keys rise by
+// ds_max_u64, and after each group the lane holding the bin's key writes its
+// value, so the table always pairs the largest |z|^2 (lowest lag among equals)
+// with its own z.  Only the final per-bin result leaves the chip.
 //
 // Reference behaviour: the same selection rule as the flat kernel
 // (src/balanced-inl.h:876-969 in the reference checkout); the reference's GPU

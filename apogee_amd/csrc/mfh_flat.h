@@ -473,6 +473,12 @@ __device__ __forceinline__ void first_twiddles(cf *w, int t, const cf *tw) {
 // would need, the spectra leave the caches: n = 65536, 4 x 128 pairs, 289 us).
 // Against a launch of its own for the merge, the same pairs take 104.8 us instead of
 // 102.6 + 10.9, most of which were the results' way to host memory.
+//
+// The order of an entry before its part's count is the machine's, not the
+// language's: these stores are relaxed, and part_is_last waits for them by
+// s_waitcnt vmcnt(0), which on gfx950 returns once a device-scope (sc1) store is
+// past the L2 and so visible to every XCD; the readers' loads are issued after
+// the count has come back.
 __device__ __forceinline__ void part_put(uint64_t *p, uint64_t x) {
   __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

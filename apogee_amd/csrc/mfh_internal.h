@@ -71,9 +71,9 @@ struct Ctx {
   // pinned host word that a hierarchical call's (or series') survivor count is
   // left in for the host, and the device word that a series sums it in
   long long *refined_host = nullptr;
-  // Whether the previous call with a count refined 1/64 of its pairs or more:
-  // the one-launch screens then cut their tiles for survivors that share a data
-  // row.  Any tile gives the same results.
+  // Whether the previous call with a count refined at least 1/64 of the coming
+  // call's pairs: the one-launch screens then cut their tiles for survivors that
+  // share a data row.  Any tile gives the same results.
   long long last_refined = 0;
   bool many_refined(long long pairs) const { return last_refined * 64 >= pairs; }
   // Per-pass twiddle tables of the flat kernel for length n (FP64-generated
@@ -309,7 +309,7 @@ struct RefinedOut {
 int hier_run(Ctx *c, int d0, int nd, int t0, int nt, size_t binsize, float threshold, size_t ws, size_t we,
              float coarse_thr, const PeakOut &out, RefinedOut count, const cf *data_rows,
              const HierScratch *hs = nullptr);
-// The survivor count that RefinedOut::kHost left (after a stream wait).
+// The survivor count of a run with RefinedOut::host set (after a stream wait).
 inline long long refined_count(const Ctx *c) { return *(volatile long long *)c->refined_host; }
 
 }  // namespace mfh

@@ -12,7 +12,7 @@
 // Exchanges go through LDS one component at a time: the real parts of all
 // points, then the imaginary parts through the same space (4.25 n bytes per
 // local point count instead of 8.5).  That is what lets two workgroups of 512
-// threads share a CU at n = 16384 and 32768 (70 KiB each), so that one computes
+// threads share a CU at n = 16384 and 32768 (68 KiB each), so that one computes
 // while the other waits at a barrier or for its rows; with 16 points per
 // thread and both components at once one workgroup of 1024 threads filled the
 // CU and every phase was exposed (n = 16384, 16 x 256: 157 us, now 104).
@@ -27,7 +27,7 @@
 // 65536, whose product is formed twice), i.e. 16 k clocks per pair and CU at
 // n = 16384 against 15.6 k waiting at nothing; measured 16.8 k (104 us for
 // 4096 pairs).  At n = 65536 one workgroup of 1024 threads fills the CU
-// (139 KiB of LDS), and loads, exchanges and arithmetic overlap only within
+// (136 KiB of LDS), and loads, exchanges and arithmetic overlap only within
 // it: 36 k of 59 k clocks issue.  Measured against the kernels before (us,
 // threshold 5.5, one filter's buffers warm): n = 8192 16 x 256: 89 to 50;
 // 16384 16 x 256: 157 to 104; 32768 4 x 256: 118 to 74; 65536 4 x 128: 120 to
@@ -771,12 +771,12 @@ bool wide_takes(const Ctx *c, size_t n, const FlatRun &r) {
   if (n < 8192 || n > 65536 || c->wide == 2) return false;
   if (c->wide == 1) return true;
   long long pairs = r.list ? (long long)r.list_cap : (long long)r.nd * r.nt;
-  // a list's length as of the previous call (results never depend on it); a
-  // captured or allocation-free call must find the buffers of the route that
-  // it takes, so it goes by the list's capacity
   // without a threshold and with several bins every sample is a candidate, which
   // costs a thread with 32 of them more
   const bool multi = r.we - r.ws > r.binsize, dense = multi && !(r.threshold > 0.f);
+  // a list's length as of the previous call (results never depend on it); a
+  // captured or allocation-free call must find the buffers of the route that
+  // it takes, so it goes by the list's capacity
   if (r.list && r.hint && !c->capturing && !c->no_alloc) {
     pairs = std::min<long long>(pairs, std::max(0, (int)*(volatile int *)r.hint));
     // the two-kernel path launches every chunk that the list could fill: 65536, 640
